@@ -232,7 +232,7 @@ vmps_status vmps_plan_time_hxv(vmps_plan* plan, int warmup, int iters, double* m
  *              use the LDS-staged 128 x 128 workgroup tiles, the rest
  *              32 x 32 wave tiles (0 = none use the big tiles);
  *   big_min64: FP64 / FP32 only: problems with both dimensions >= big_min64
- *              use LDS-staged 128 x 128 workgroup tiles (0 = none, the default);
+ *              use LDS-staged 64 x 64 or 128 x 128 workgroup tiles (0 = none);
  *   explicit_u: 0 = the combine U = sum c T is done on stage C's operand
  *              load (U never stored); 1 = a separate kernel forms U once per
  *              (output block, R block) and stage C reads it (pays off when
@@ -248,8 +248,8 @@ typedef struct {
 } vmps_tile_config;
 
 vmps_status vmps_plan_get_tiles(const vmps_plan* plan, vmps_tile_config* cfg);
-/* Results do not depend on the configuration beyond FP rounding of the
- * split-BF16 path (FP64: bit-identical sums in the same order per tile). */
+/* Results do not depend on the configuration beyond the rounding of sums
+ * taken in another order. */
 vmps_status vmps_plan_set_tiles(vmps_plan* plan, const vmps_tile_config* cfg);  /* ms .. n_tried ignored */
 /* Autotuner: times every candidate configuration of the plan's precision
  * (`iters` HxV each on the plan's resident vectors) and keeps the fastest.

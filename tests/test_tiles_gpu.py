@@ -134,3 +134,53 @@ def test_fp64_fp32_big_tiles(case, precision, tol, big_min64, xu):
     cfg = H.tiles()
     assert cfg["big_min64"] == big_min64 and cfg["explicit_u"] == xu
     assert _rel(HxV(H, v), ref) <= tol
+
+
+# sector dimensions at the edges of the 16 x 16 accumulators, 32-row steps, 16-deep K
+# steps and 64-wide tiles of the LDS-staged kernels, odd ones among them
+EDGE_LEFT = [((-5,), 1), ((-3,), 17), ((-1,), 64), ((1,), 65), ((3,), 33), ((5,), 130), ((7,), 2)]
+EDGE_RIGHT = [((-5,), 3), ((-3,), 16), ((-1,), 127), ((1,), 31), ((3,), 96), ((5,), 48), ((7,), 15)]
+
+
+@pytest.fixture(scope="module")
+def edge_case():
+    from vmps_amd import models
+    W = models.heisenberg_u1_mpo()
+    pd = synth.make_pivot(W, W, EDGE_LEFT, EDGE_RIGHT, np.random.default_rng(12))
+    v = synth.random_vector(pd, 13)
+    lib = oracle.load()
+    h = pivots.build_oracle(lib, pd)
+    try:
+        return pd, v, pivots.oracle_hxv(lib, h, v, nthreads=8)
+    finally:
+        lib.oracle_pivot2_destroy(h)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", FP64_RTOL), ("fp32", 1e-5)])
+@pytest.mark.parametrize("big_min64,xu", [(1, 1), (1, 0), (33, 1)])
+def test_lds_tiles_at_block_edges(edge_case, precision, tol, big_min64, xu):
+    pd, v, ref = edge_case
+    print("LDS tiles at edges", precision, big_min64, xu, flush=True)
+    H = PivotMatrix2(pd, precision=precision)
+    H.set_tiles(big_min64=big_min64, explicit_u=xu)
+    assert _rel(HxV(H, v), ref) <= tol
+
+
+@pytest.mark.parametrize("M,nleft", [(640, 29), (2047, 30)])
+def test_lds_tiles_split_k(M, nleft):
+    """Stage C tiles cut along K, in 64-wide (M = 640) and 128-wide (M = 2047)
+    tiles, against the wave tiles: both sum a few thousand products per element
+    in FP64, so they agree to 1e-13 of the result's norm."""
+    from vmps_amd import models
+    W = models.heisenberg_su2_lr_mpo(synth.lr_couplings(3, np.random.default_rng(1)))
+    pd = synth.make_pivot(W, W, synth.heisenberg_su2_bond(nleft, M), synth.heisenberg_su2_bond(nleft + 2, M),
+                          np.random.default_rng(14))
+    v = synth.random_vector(pd, 15)
+    print("split K", M, "vsize", pd.vsize, flush=True)
+    H = PivotMatrix2(pd)
+    H.set_tiles(big_min64=0, explicit_u=0)
+    ref = HxV(H, v)
+    H.set_tiles(big_min64=1, explicit_u=1)
+    out = HxV(H, v)
+    assert _rel(out, ref) <= 1e-13
+    assert np.array_equal(HxV(H, v), out)  # a fixed order of summation

@@ -732,11 +732,13 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
     return (double)ms / iters;
   };
   TileChoice pick{D.H.wave_edge, D.H.big_min, D.H.big_min64, D.H.explicit_u};
-  // Pivots with blocks of 256 and more always take the FP64 / FP32 big tiles:
-  // without them such a pivot's HxV is 2-3x slower (C60 at M = 4096: 124 ms
-  // against 45 ms), so the search neither starts from nor times that choice.
+  // Pivots with blocks of 256 and more keep the FP64 / FP32 LDS-staged tiles
+  // with the explicit stage B, which their plans start from: wave tiles take
+  // 1.3 to 2.5 times as long (C60 at M = 4096: 58 against 24 ms; U(1) chain at
+  // M = 2048: 339 against 263 us), the fused stage B 1.1 to 1.3 times.
   const bool large = D.H.stats.max_block_dim >= 2 * vmps::kBigTile && D.prec != VMPS_PREC_BF16X3;
-  if (large && pick.big_min64 <= 0) pick.big_min64 = vmps::kBigTile;
+  if (large && pick.big_min64 <= 0) pick.big_min64 = 1;
+  if (large) pick.explicit_u = true;
   double best = measure(pick);
   int tried = 1;
   auto consider = [&](TileChoice c) {
@@ -757,20 +759,19 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
       c.big_min = b;
       consider(c);
     }
-  } else {
+  } else if (!large) {
     for (int e : {16, 32}) {
       TileChoice c = pick;
       c.wave_edge = e;
       consider(c);
     }
-    for (int b64 : {0, vmps::kBigTile}) {
-      if (large && b64 == 0) continue;
-      TileChoice c = pick;
-      c.big_min64 = b64;
-      consider(c);
-    }
+    TileChoice c = pick;  // every problem on the LDS-staged tiles, U formed once
+    c.big_min64 = 1;
+    c.explicit_u = true;
+    consider(c);
   }
   for (bool xu : {false, true}) {
+    if (large && !xu) continue;
     TileChoice c = pick;
     c.explicit_u = xu;
     consider(c);

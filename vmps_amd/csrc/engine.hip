@@ -271,217 +271,392 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
   }
 }
 
-// ---- LDS-staged 128 x 128 workgroup tiles for large blocks ------------------
-// The big-tile kernels ask for two waves per SIMD (amdgpu_waves_per_eu): the
-// compiler then keeps accumulators and operands within 256 registers (no
-// spills) instead of using up to 384, and two workgroups share a CU.
-// Problems with both dimensions >= H.big_min64 (a tile configuration choice,
-// off by default).  4 waves in a 2 x 2 grid, each owning 64 x 64 = 4 x 4 MFMA
-// accumulators.  Per 16-deep K step the workgroup
-// stages A[128 x 16] and B[16 x 128] k-major in LDS (the layout the MFMA
-// lanes read: 16 consecutive rows / columns per k) with coalesced global
-// loads, so every operand element is fetched from HBM once per tile instead
-// of once per 16- or 32-wide wave tile.  The next K step's global loads are
-// issued before the MFMAs of the current one.
-constexpr int kBT = kBigTile;
+// ---- LDS-staged BT x BT workgroup tiles for large blocks (BT = 64 or 128) ------
+// Problems with both dimensions >= H.big_min64.  4 waves in a 2 x 2 grid; per
+// 16-deep K step the workgroup stages A[BT x 16] and B[16 x BT] k-major in LDS
+// (the layout the MFMA lanes read: 16 consecutive rows / columns per k), two
+// buffers, so every operand element is fetched once per tile and a step has one
+// barrier.
+//
+// What bounds it: the FP64 MFMA (16x16x4, 64 cycles).  A wave issues in order, so
+// every memory instruction that is not between two MFMAs, and every mask and
+// address computation, is time the matrix core waits (a batch of 24 products of
+// 1024^3: 70.6 TFLOP/s without any staging, 56 with the loads and LDS writes of a
+// step issued together, 64 with one between every two MFMAs).  Hence:
+//  - rows and columns past the block's edge are clamped to its last one (their
+//    results are not stored), offsets are fixed per thread and the K step moves
+//    the wave-uniform buffer descriptor, whose range returns zeros past K;
+//  - the sub-blocks of a tile are dealt to the waves alternately (row
+//    32 x + 16 (wave % 2) + lane % 16, columns likewise) and a tile at the edge runs
+//    the NX x NY instance that covers it: it costs in steps of 32 rows and columns
+//    instead of BT (C60 at M = 4096: 5% padding work instead of 22%);
+//  - a step is scheduled as four slices of NX NY MFMAs with the LDS reads of the
+//    next slice, the LDS writes of the next step and the loads of the step after
+//    that in between.
 constexpr int kBKd = 16;
-constexpr int kBQ = kBKd / 2;  // K elements each thread stages per operand and step
 
 template <class T>
-struct BigTileSmem {
-  T A[kBKd][kBT];
-  T B[kBKd][kBT];
+struct RawLoad;
+template <>
+struct RawLoad<double> {
+  typedef double v2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static double one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
+  }
+  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
+    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b128(r, v, 0, 0));
+  }
+};
+template <>
+struct RawLoad<float> {
+  typedef float v2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static float one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
+  }
+  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
+    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b64(r, v, 0, 0));
+  }
+};
+template <class T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const T* p, int elems) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), (short)0, elems * (int)sizeof(T), 0x00020000);
+}
+
+// Staging state of a workgroup: the tile, the operands of the load cursor, and
+// the elements a thread has in flight.
+template <class T, int BT>
+struct BigTile {
+  static constexpr int S = BT / 32;            // 16 x 16 accumulators per wave and dimension
+  static constexpr int kNA = kBKd * BT / 256;  // A elements per thread and step
+  static constexpr int kNB = kNA / 2;          // B pairs per thread and step
+  static constexpr int kDA = 256 / BT;         // k distance of a thread's A elements
+  // LDS rows start on other banks (64 of 4 bytes) so that neither the reads (16
+  // consecutive elements of 4 rows) nor the writes of B's pairs (rows k, k + 2,
+  // .. k + 14 of 8 columns) collide: element (k, i) of B at row_b(k) + i
+  static constexpr int kPad = 256 / (int)sizeof(T);
+  static constexpr int kRow = BT + kPad;
+  __device__ __forceinline__ static int row_a(int k) { return k * kRow + (16 * (k & 1) & (kPad - 1)); }
+  __device__ __forceinline__ static int row_b(int k) {
+    const int s = sizeof(T) == 8 ? 16 * (k & 1) + 8 * ((k >> 1) & 1) + 16 * ((k >> 2) & 1)
+                                 : 16 * (k & 3) + 8 * ((k >> 2) & 1);
+    return k * kRow + (s & (kPad - 1));
+  }
+  struct Smem {  // FP64, BT = 128: 80 KB, two workgroups fill a CU's 160 KB
+    T A[2][kBKd * kRow];
+    T B[2][kBKd * kRow];
+  };
+  typedef typename RawLoad<T>::v2 pair_t;
+
+  T ra[kNA];
+  pair_t rb[kNB];
+  uint32_t offA, offB[kNB];
+  const T *A, *B;      // wave-uniform: k = 0 of the tile's first row / column
+  int M, N, K, m0, n0;
+  int ai, ak, bj, bk;  // staging roles: A row and first k, B column and first k
+  int wm, wn, li, lk;  // wave's first row / column, lane's row and k
+
+  __device__ __forceinline__ void init(int M_, int N_, int mt, int nt, int tid) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    M = M_;
+    N = N_;
+    m0 = mt * BT;
+    n0 = nt * BT;
+    li = lane & 15;
+    lk = lane >> 4;
+    wm = (wave & 1) * 16;
+    wn = (wave >> 1) * 16;
+    ai = tid % BT;
+    ak = tid / BT;
+    bj = tid >> 3;
+    bk = (tid & 7) * 2;
+    offA = (uint32_t)sizeof(T) * (uint32_t)(ak * M + min(ai, M - 1 - m0));
+  }
+  __device__ __forceinline__ int nx() const { return min(S, (M - m0 + 31) / 32); }  // workgroup-uniform
+  __device__ __forceinline__ int ny() const { return min(S, (N - n0 + 31) / 32); }
+  // the product's operands and K extent (a chunk of stage C, stage A's blocks)
+  __device__ __forceinline__ void set(const T* Ablk, const T* Bblk, int K_) {
+    K = K_;
+    A = Ablk + m0;
+    B = Bblk + (int64_t)n0 * K;
+#pragma unroll
+    for (int h = 0; h < kNB; ++h)
+      offB[h] = (uint32_t)sizeof(T) * (uint32_t)(min(bj + 32 * h, N - 1 - n0) * K + bk);
+  }
+  // K step at kb; nothing is read past K (A by the buffer's range, B by an
+  // offset beyond it), and with kb >= K the loads return zeros
+  __device__ __forceinline__ void load_a(int kb) {
+    const auto r = raw_buffer(A + (int64_t)kb * M, max(0, min(K - kb, kBKd) * M - m0));
+#pragma unroll
+    for (int q = 0; q < kNA; ++q)
+      ra[q] = RawLoad<T>::one(r, offA, (uint32_t)sizeof(T) * (uint32_t)(kDA * q * M));
+  }
+  __device__ __forceinline__ void load_b(int kb) {
+    const auto r = raw_buffer(B + kb, kb < K ? 0x7fffffff / (int)sizeof(T) : 0);
+    const bool in0 = kb + bk < K, in1 = kb + bk + 1 < K;
+#pragma unroll
+    for (int h = 0; h < kNB; ++h) {
+      rb[h] = RawLoad<T>::two(r, in0 ? offB[h] : 0x80000000u);
+      if (!in1) rb[h][1] = T(0);
+    }
+  }
+  __device__ __forceinline__ void stage(Smem& s, int buf) const {
+#pragma unroll
+    for (int q = 0; q < kNA; ++q) s.A[buf][row_a(ak + kDA * q) + ai] = ra[q];
+#pragma unroll
+    for (int h = 0; h < kNB; ++h) {
+      s.B[buf][row_b(bk) + bj + 32 * h] = rb[h][0];
+      s.B[buf][row_b(bk + 1) + bj + 32 * h] = rb[h][1];
+    }
+  }
 };
 
-template <class T>
-__device__ inline void big_tile_mac(const BigTileSmem<T>& s, int wm, int wn, int li, int lk,
-                                    typename Mfma<T>::acc_t (&acc)[4][4]) {
-#pragma unroll
-  for (int ks = 0; ks < kBKd; ks += 4) {
-    T a[4], b[4];
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      a[x] = s.A[ks + lk][wm + 16 * x + li];
-      b[x] = s.B[ks + lk][wn + 16 * x + li];
-    }
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) Mfma<T>::mac(b[y], a[x], acc[x][y]);
-  }
-}
+// NX x NY accumulators of 16 x 16 per wave over `steps` K steps.  next(g) moves
+// the load cursor to the following step and issues its loads.
+template <class T, int BT, int NX, int NY>
+struct BigAcc {
+  typedef BigTile<T, BT> Tile;
+  typedef typename Mfma<T>::acc_t acc_t;
+  acc_t acc[NX][NY];
+  T a[2][NX], b[2][NY];
 
-template <class T, class OutT>
-__device__ inline void big_tile_store(OutT* __restrict__ C, int M, int N, int m0, int n0, int lane,
-                                      const typename Mfma<T>::acc_t (&acc)[4][4]) {
+  __device__ __forceinline__ void zero() {
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int i = m0 + 16 * x + (lane & 15);
-    if (i >= M) continue;
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int j = n0 + 16 * y + Mfma<T>::col(lane, v);
-        if (j < N) C[(int64_t)j * M + i] = (OutT)acc[x][y][v];
-      }
+      for (int y = 0; y < NY; ++y) acc[x][y] = acc_t{0, 0, 0, 0};
   }
-}
-
-// Thread roles in the staging loads (256 threads, 2048 elements per operand):
-//   A (column-major, ld M): row i = tid % 128, k = kb + tid/128 + 2q, q < kBQ
-//   B (column-major K x N, ld K): column j = tid / 2, k = kb + kBQ (tid % 2) + q
-template <class T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_a_big(const TileA* __restrict__ tiles, int ntiles,
-                                                     const T* __restrict__ L, const T* __restrict__ V,
-                                                     T* __restrict__ Tout) {
-  __shared__ BigTileSmem<T> s;
-  if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-  const TileA t = tiles[blockIdx.x];
-  const int m0 = t.mt * kBT, n0 = t.nt * kBT;
-  const T* __restrict__ A = L + t.a_off;
-  const T* __restrict__ B = V + t.b_off;
-  const int ai = tid & 127, ak = tid >> 7, bj = tid >> 1, bk = (tid & 1) * kBQ;
-  const bool arow = m0 + ai < t.M, bcol = n0 + bj < t.N;
-  typename Mfma<T>::acc_t acc[4][4];
+  __device__ __forceinline__ void read(const Tile& g, const typename Tile::Smem& s, int buf, int ks, int p) {
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < NX; ++x) a[p][x] = s.A[buf][Tile::row_a(ks + g.lk) + g.wm + 32 * x + g.li];
 #pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = typename Mfma<T>::acc_t{0, 0, 0, 0};
-  T ra[kBQ], rb[kBQ];
-  auto gload = [&](int kb) {
+    for (int y = 0; y < NY; ++y) b[p][y] = s.B[buf][Tile::row_b(ks + g.lk) + g.wn + 32 * y + g.li];
+  }
+  __device__ __forceinline__ void mac(int p) {
 #pragma unroll
-    for (int q = 0; q < kBQ; ++q) {
-      const int ka = kb + ak + 2 * q, kbb = kb + bk + q;
-      ra[q] = (arow && ka < t.K) ? A[(int64_t)ka * t.M + m0 + ai] : T(0);
-      rb[q] = (bcol && kbb < t.K) ? B[(int64_t)(n0 + bj) * t.K + kbb] : T(0);
+    for (int y = 0; y < NY; ++y)
+#pragma unroll
+      for (int x = 0; x < NX; ++x) Mfma<T>::mac(b[p][y], a[p][x], acc[x][y]);
+  }
+  // schedule of a slice: an LDS read, an LDS write or a load after each MFMA
+  template <int kReads, int kWrites, int kLoads>
+  __device__ __forceinline__ static void interleave() {
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
     }
-  };
-  gload(0);
-  for (int kb = 0; kb < t.K; kb += kBKd) {
-    __syncthreads();  // the previous step's LDS reads are done
 #pragma unroll
-    for (int q = 0; q < kBQ; ++q) {
-      s.A[ak + 2 * q][ai] = ra[q];
-      s.B[bk + q][bj] = rb[q];
+    for (int i = 0; i < kWrites; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
     }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // global load
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  template <class Next>
+  __device__ __forceinline__ void run(Tile& g, typename Tile::Smem& s, int steps, Next&& next) {
+    constexpr int kR = (NX + 1) / 2 + (NY + 1) / 2, kW = Tile::kNA / 2 + Tile::kNB, kL = Tile::kNA + Tile::kNB;
+    zero();
+    if (steps <= 0) return;  // workgroup-uniform
+    next(g);
+    g.stage(s, 0);
+    next(g);
     __syncthreads();
-    if (kb + kBKd < t.K) gload(kb + kBKd);
-    big_tile_mac<T>(s, wm, wn, li, lk, acc);
+    read(g, s, 0, 0, 0);
+    for (int buf = 0; steps > 0; --steps, buf ^= 1) {
+      __builtin_amdgcn_sched_barrier(0);
+      read(g, s, buf, 4, 1);
+      g.stage(s, buf ^ 1);
+      mac(0);
+      interleave<kR, kW, 0>();
+      read(g, s, buf, 8, 0);
+      next(g);
+      mac(1);
+      interleave<kR, 0, kL>();
+      read(g, s, buf, 12, 1);
+      mac(0);
+      interleave<kR, 0, 0>();
+      __syncthreads();  // the other buffer is staged, and this one no longer read
+      __builtin_amdgcn_sched_barrier(0);
+      read(g, s, buf ^ 1, 0, 0);
+      mac(1);
+      interleave<kR, 0, 0>();
+    }
   }
-  big_tile_store<T, T>(Tout + t.c_off, t.M, t.N, m0 + wm, n0 + wn, lane, acc);
+  // into C (ld ldc), at the tile's corner; rows and columns past the block are dropped
+  template <class OutT>
+  __device__ __forceinline__ void store(const Tile& g, OutT* __restrict__ C, int64_t ldc) const {
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+      const int r = g.wm + 32 * x + g.li;
+      if (g.m0 + r >= g.M) continue;
+#pragma unroll
+      for (int y = 0; y < NY; ++y)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int c = g.wn + 32 * y + Mfma<T>::col(16 * g.lk, v);
+          if (g.n0 + c < g.N) C[c * ldc + r] = (OutT)acc[x][y][v];
+        }
+    }
+  }
+};
+
+// f(BigAcc of the instance covering the tile); workgroup-uniform
+template <class T, int BT, class F>
+__device__ __forceinline__ void with_big_acc(const BigTile<T, BT>& g, F&& f) {
+  const int nx = g.nx(), ny = g.ny();
+#define VMPS_BIG_ACC(X, Y)                                   \
+  if constexpr (X <= BigTile<T, BT>::S && Y <= BigTile<T, BT>::S) \
+    if (nx == X && ny == Y) {                                \
+      BigAcc<T, BT, X, Y> acc;                               \
+      f(acc);                                                \
+      return;                                                \
+    }
+#define VMPS_BIG_ACC_ROW(X) VMPS_BIG_ACC(X, 1) VMPS_BIG_ACC(X, 2) VMPS_BIG_ACC(X, 3) VMPS_BIG_ACC(X, 4)
+  VMPS_BIG_ACC_ROW(1)
+  VMPS_BIG_ACC_ROW(2)
+  VMPS_BIG_ACC_ROW(3)
+  VMPS_BIG_ACC_ROW(4)
+#undef VMPS_BIG_ACC_ROW
+#undef VMPS_BIG_ACC
+}
+
+// Stage A, large blocks: T (M x N, ld M) = L (M x K, ld M) . V (K x N, ld K).
+template <class T, int BT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_a_big(
+    const TileA* __restrict__ tiles, int ntiles, const T* __restrict__ L, const T* __restrict__ V,
+    T* __restrict__ Tout) {
+  __shared__ typename BigTile<T, BT>::Smem s;
+  if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
+  const TileA t = tiles[blockIdx.x];
+  if (t.K <= 0) return;  // a padding slot of the launch order (workgroup-uniform)
+  BigTile<T, BT> g;
+  g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
+  g.set(L + t.a_off, V + t.b_off, t.K);
+  with_big_acc(g, [&](auto& acc) {
+    int kb = 0;
+    acc.run(g, s, (t.K + kBKd - 1) / kBKd, [&](BigTile<T, BT>& h) {
+      h.load_a(kb);
+      h.load_b(kb);
+      kb += kBKd;
+    });
+    acc.store(g, Tout + t.c_off + (int64_t)g.n0 * t.M + g.m0, t.M);
+  });
 }
 
 // Stage C, large output blocks: Vout = sum over chunks (sum_j c_j T_j) . R_r.
-// The combine U = sum c_j T_j is formed while staging the A operand: the
-// chunk's term list is loaded once per lane and broadcast with readlane.
-// kOneTerm: every chunk has exactly one term (explicit stage B), which the
-// kernel then streams with the next K step's loads in flight; a separate
-// instantiation, so that the general path's registers do not add up with it.
-template <class T, class OutT, bool kOneTerm>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_big(const TileC* __restrict__ tiles, int ntiles,
-                                                     const ChunkC* __restrict__ chunks,
-                                                     const TermC* __restrict__ terms, const T* __restrict__ Tbuf,
-                                                     const T* __restrict__ R, OutT* __restrict__ Vout) {
-  __shared__ BigTileSmem<T> s;
-  if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-  const TileC t = tiles[blockIdx.x];
-  const int m0 = t.mt * kBT, n0 = t.nt * kBT;
-  const int ai = tid & 127, ak = tid >> 7, bj = tid >> 1, bk = (tid & 1) * kBQ;
-  const bool arow = m0 + ai < t.M, bcol = n0 + bj < t.N;
-  typename Mfma<T>::acc_t acc[4][4];
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = typename Mfma<T>::acc_t{0, 0, 0, 0};
-  for (int c = t.chunk_begin; c < t.chunk_end; ++c) {
-    const ChunkC ch = chunks[c];
-    const int K = ch.K;
-    const T* __restrict__ B = R + ch.r_off;
-    const int nt = ch.term_end - ch.term_begin;
-    int64_t my_toff = 0;
-    T my_c = T(0);
-    if (lane < nt) {
-      const TermC tm = terms[ch.term_begin + lane];
-      my_toff = tm.t_off;
-      my_c = (T)tm.c;
-    }
-    if (kOneTerm) {  // one term (explicit stage B): a plain product, next step's loads in flight
-      const T* __restrict__ T0 = Tbuf + readlane64(my_toff, 0);
-      const T c0 = readlane_t<T>(my_c, 0);
-      T ra[kBQ], rb[kBQ];
-      auto gload = [&](int kb) {
-#pragma unroll
-        for (int q = 0; q < kBQ; ++q) {
-          const int ka = kb + ak + 2 * q, kbb = kb + bk + q;
-          ra[q] = (arow && ka < K) ? T0[(int64_t)ka * t.M + m0 + ai] : T(0);
-          rb[q] = (bcol && kbb < K) ? B[(int64_t)(n0 + bj) * K + kbb] : T(0);
+// A work item is a run of K steps of one tile (BigItemC): the whole tile, or
+// with slot >= 0 a part of it, whose BT x BT partial sums k_reduce_big adds up
+// in slot order.
+// kOneTerm: every chunk reads one stored block of unit weight (explicit stage
+// B), and the loads run ahead across the chunks' boundaries.  Otherwise the
+// combine U = sum c_j T_j is formed on the operand load, the chunk's term list
+// loaded once per lane and broadcast with readlane.
+template <class T, class OutT, int BT, bool kOneTerm>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_big(
+    const TileC* __restrict__ tiles, const BigItemC* __restrict__ items, int nitems,
+    const ChunkC* __restrict__ chunks, const TermC* __restrict__ terms, const T* __restrict__ Tbuf,
+    const T* __restrict__ R, OutT* __restrict__ Vout, T* __restrict__ partial) {
+  typedef BigTile<T, BT> Tile;
+  __shared__ typename Tile::Smem s;
+  if ((int)blockIdx.x >= nitems) return;  // workgroup-uniform
+  const BigItemC w = items[blockIdx.x];
+  if (w.tile < 0) return;  // a padding slot of the launch order (workgroup-uniform)
+  const TileC t = tiles[w.tile];
+  Tile g;
+  g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
+  int left = w.nsteps, c = w.chunk, kb = w.step * kBKd;
+  auto out = [&](auto& acc) __attribute__((always_inline)) {
+    if (w.slot < 0)
+      acc.store(g, Vout + t.c_off + (int64_t)g.n0 * t.M + g.m0, t.M);
+    else
+      acc.store(g, partial + w.slot * (int64_t)(BT * BT), BT);
+  };
+  if constexpr (kOneTerm) {
+    auto enter = [&](Tile& h) __attribute__((always_inline)) {
+      const ChunkC ch = chunks[c];
+      h.set(Tbuf + terms[ch.term_begin].t_off, R + ch.r_off, ch.K);
+    };
+    if (left > 0) enter(g);
+    with_big_acc(g, [&](auto& acc) __attribute__((always_inline)) {
+      acc.run(g, s, w.nsteps, [&](Tile& h) __attribute__((always_inline)) {
+        while (kb >= h.K && left > 0) {
+          ++c;
+          kb = 0;
+          enter(h);
         }
-      };
-      gload(0);
-      for (int kb = 0; kb < K; kb += kBKd) {
+        --left;
+        h.load_a(kb);
+        h.load_b(kb);
+        kb += kBKd;
+      });
+      out(acc);
+    });
+  } else {
+    const int lane = threadIdx.x & 63;
+    BigAcc<T, BT, Tile::S, Tile::S> acc;
+    acc.zero();
+    for (; left > 0; ++c, kb = 0) {
+      const ChunkC ch = chunks[c];
+      const int nt = ch.term_end - ch.term_begin;
+      int64_t my_toff = 0;
+      T my_c = T(0);
+      if (lane < nt) {
+        const TermC tm = terms[ch.term_begin + lane];
+        my_toff = tm.t_off;
+        my_c = (T)tm.c;
+      }
+      g.set(Tbuf, R + ch.r_off, ch.K);
+      for (; kb < ch.K && left > 0; kb += kBKd, --left) {
+        T u[Tile::kNA];
+#pragma unroll
+        for (int q = 0; q < Tile::kNA; ++q) u[q] = T(0);
+        g.load_b(kb);
+        for (int jt = 0; jt < nt; ++jt) {
+          g.A = Tbuf + readlane64(my_toff, jt) + g.m0;
+          g.load_a(kb);
+          const T c0 = readlane_t<T>(my_c, jt);
+#pragma unroll
+          for (int q = 0; q < Tile::kNA; ++q) u[q] += c0 * g.ra[q];
+        }
+#pragma unroll
+        for (int q = 0; q < Tile::kNA; ++q) g.ra[q] = u[q];
         __syncthreads();  // the previous step's LDS reads are done
-#pragma unroll
-        for (int q = 0; q < kBQ; ++q) {
-          s.A[ak + 2 * q][ai] = c0 * ra[q];
-          s.B[bk + q][bj] = rb[q];
-        }
+        g.stage(s, 0);
         __syncthreads();
-        if (kb + kBKd < K) gload(kb + kBKd);
-        big_tile_mac<T>(s, wm, wn, li, lk, acc);
-      }
-      continue;
-    }
-    for (int kb = 0; kb < K; kb += kBKd) {
-      T ra[kBQ], rb[kBQ];
 #pragma unroll
-      for (int q = 0; q < kBQ; ++q) {
-        const int kbb = kb + bk + q;
-        rb[q] = (bcol && kbb < K) ? B[(int64_t)(n0 + bj) * K + kbb] : T(0);
-        ra[q] = T(0);
-      }
-      int jt = 0;
-      for (; jt + 1 < nt; jt += 2) {
-        const T* __restrict__ T0 = Tbuf + readlane64(my_toff, jt);
-        const T* __restrict__ T1 = Tbuf + readlane64(my_toff, jt + 1);
-        const T c0 = readlane_t<T>(my_c, jt), c1 = readlane_t<T>(my_c, jt + 1);
-        T x0[kBQ], x1[kBQ];
-#pragma unroll
-        for (int q = 0; q < kBQ; ++q) {
-          const int ka = kb + ak + 2 * q;
-          const bool ok = arow && ka < K;
-          x0[q] = ok ? T0[(int64_t)ka * t.M + m0 + ai] : T(0);
-          x1[q] = ok ? T1[(int64_t)ka * t.M + m0 + ai] : T(0);
-        }
-#pragma unroll
-        for (int q = 0; q < kBQ; ++q) ra[q] += c0 * x0[q] + c1 * x1[q];
-      }
-      if (jt < nt) {
-        const T* __restrict__ T0 = Tbuf + readlane64(my_toff, jt);
-        const T c0 = readlane_t<T>(my_c, jt);
-#pragma unroll
-        for (int q = 0; q < kBQ; ++q) {
-          const int ka = kb + ak + 2 * q;
-          ra[q] += c0 * ((arow && ka < K) ? T0[(int64_t)ka * t.M + m0 + ai] : T(0));
+        for (int ks = 0; ks < kBKd; ks += 4) {
+          acc.read(g, s, 0, ks, 0);
+          acc.mac(0);
         }
       }
-      __syncthreads();  // the previous step's LDS reads are done
-#pragma unroll
-      for (int q = 0; q < kBQ; ++q) {
-        s.A[ak + 2 * q][ai] = ra[q];
-        s.B[bk + q][bj] = rb[q];
-      }
-      __syncthreads();
-      big_tile_mac<T>(s, wm, wn, li, lk, acc);
     }
+    out(acc);
   }
-  big_tile_store<T, OutT>(Vout + t.c_off, t.M, t.N, m0 + wm, n0 + wn, lane, acc);
+}
+
+// Vout tile = sum over its split partials, in slot order; one workgroup per
+// quarter of a tile's columns.
+template <class T, class OutT, int BT>
+__global__ __launch_bounds__(256) void k_reduce_big(const TileC* __restrict__ tiles, const BigRedC* __restrict__ reds,
+                                                    const T* __restrict__ partial, OutT* __restrict__ Vout) {
+  const BigRedC r = reds[blockIdx.x / 4];
+  const TileC t = tiles[r.tile];
+  const int i = t.mt * BT + threadIdx.x % BT;
+  if (i >= t.M) return;
+  const int c0 = (int)(blockIdx.x % 4) * (BT / 4) + threadIdx.x / BT;
+  for (int c = c0; c < (int)(blockIdx.x % 4 + 1) * (BT / 4); c += 256 / BT) {
+    const int j = t.nt * BT + c;
+    if (j >= t.N) return;
+    const T* p = partial + r.slot * (int64_t)(BT * BT) + c * BT + threadIdx.x % BT;
+    T acc = p[0];
+    for (int q = 1; q < r.nsplit; ++q) acc += p[(int64_t)q * (BT * BT)];
+    Vout[t.c_off + (int64_t)j * t.M + i] = (OutT)acc;
+  }
 }
 
 // Weighted dot product, pass 1: workgroup b reduces segments [b*spb, (b+1)*spb).
@@ -683,6 +858,10 @@ void DevPlan::upload_lists() {
   tilesC.upload(H.tilesC_w, stream);
   tilesAb.upload(H.tilesA_b, stream);  // FP64 / FP32 big-tile kernels
   tilesCb.upload(H.tilesC_b, stream);
+  itemsCb.upload(H.itemsC_b, stream);
+  redsCb.upload(H.redsC_b, stream);
+  if (partCb.n < (size_t)(H.slotsC_b * H.big_edge * H.big_edge))
+    partCb.alloc((size_t)(H.slotsC_b * H.big_edge * H.big_edge));
   chunksC.upload(H.chunksC, stream);
   termsC.upload(H.termsC, stream);
   combTasks.upload(H.comb_tasks, stream);
@@ -716,11 +895,44 @@ void DevPlan::ensure_precision_buffers() {
   if (prec == VMPS_PREC_BF16X3) ensure_bf16_buffers();
 }
 
+namespace {
+template <class T>
+void launch_a_big(DevPlan& D, const T* L, const T* V, T* Tout, hipStream_t s) {
+  const int n = (int)D.tilesAb.n;
+  if (D.H.big_edge == 64)
+    hipLaunchKernelGGL((k_stage_a_big<T, 64>), dim3(n), dim3(256), 0, s, D.tilesAb.p, n, L, V, Tout);
+  else
+    hipLaunchKernelGGL((k_stage_a_big<T, 128>), dim3(n), dim3(256), 0, s, D.tilesAb.p, n, L, V, Tout);
+}
+
+template <class T, int BT>
+void launch_c_big_edge(DevPlan& D, const T* src, const T* R, double* d_vout, hipStream_t s) {
+  const int n = (int)D.itemsCb.n, nr = (int)D.redsCb.n;
+  T* part = reinterpret_cast<T*>(D.partCb.p);
+  if (D.H.explicit_u)
+    hipLaunchKernelGGL((k_stage_c_big<T, double, BT, true>), dim3(n), dim3(256), 0, s, D.tilesCb.p, D.itemsCb.p, n,
+                       D.chunksC.p, D.termsC.p, src, R, d_vout, part);
+  else
+    hipLaunchKernelGGL((k_stage_c_big<T, double, BT, false>), dim3(n), dim3(256), 0, s, D.tilesCb.p, D.itemsCb.p, n,
+                       D.chunksC.p, D.termsC.p, src, R, d_vout, part);
+  if (nr)
+    hipLaunchKernelGGL((k_reduce_big<T, double, BT>), dim3(4 * nr), dim3(256), 0, s, D.tilesCb.p, D.redsCb.p, part,
+                       d_vout);
+}
+
+template <class T>
+void launch_c_big(DevPlan& D, const T* src, const T* R, double* d_vout, hipStream_t s) {
+  if (D.H.big_edge == 64)
+    launch_c_big_edge<T, 64>(D, src, R, d_vout, s);
+  else
+    launch_c_big_edge<T, 128>(D, src, R, d_vout, s);
+}
+}  // namespace
+
 void DevPlan::launch_stage(int stage, const double* d_vin, double* d_vout, hipStream_t s) {
-  const int nA = (int)tilesA.n, nC = (int)tilesC.n, nAb = (int)tilesAb.n, nCb = (int)tilesCb.n;
+  const int nA = (int)tilesA.n, nC = (int)tilesC.n, nAb = (int)tilesAb.n, nCb = (int)itemsCb.n;
   if (prec == VMPS_PREC_FP64) {
-    if (stage == 0 && nAb)
-      hipLaunchKernelGGL(k_stage_a_big<double>, dim3(nAb), dim3(256), 0, s, tilesAb.p, nAb, L.p, d_vin, T.p);
+    if (stage == 0 && nAb) launch_a_big<double>(*this, L.p, d_vin, T.p, s);
     if (stage == 0 && nA) {
       if (H.wave_edge == 16)
         hipLaunchKernelGGL((k_stage_a<double, 16>), dim3(grid_for(nA)), dim3(256), 0, s, tilesA.p, nA, L.p, d_vin,
@@ -737,12 +949,7 @@ void DevPlan::launch_stage(int stage, const double* d_vin, double* d_vout, hipSt
                              combTerms.p, T.p, Ub.p);
         src = Ub.p;
       }
-      if (nCb && H.explicit_u)
-        hipLaunchKernelGGL((k_stage_c_big<double, double, true>), dim3(nCb), dim3(256), 0, s, tilesCb.p, nCb,
-                           chunksC.p, termsC.p, src, R.p, d_vout);
-      else if (nCb)
-        hipLaunchKernelGGL((k_stage_c_big<double, double, false>), dim3(nCb), dim3(256), 0, s, tilesCb.p, nCb,
-                           chunksC.p, termsC.p, src, R.p, d_vout);
+      if (nCb) launch_c_big<double>(*this, src, R.p, d_vout, s);
       if (nC && H.wave_edge == 16)
         hipLaunchKernelGGL((k_stage_c<double, double, 16>), dim3(nC), dim3(256), 0, s, tilesC.p, nC, chunksC.p,
                            termsC.p, src, R.p, d_vout);
@@ -753,8 +960,7 @@ void DevPlan::launch_stage(int stage, const double* d_vin, double* d_vout, hipSt
   } else if (prec == VMPS_PREC_FP32) {
     if (stage == 0) {
       if (H.ysize) hipLaunchKernelGGL(k_f64_to_f32, dim3(1024), dim3(256), 0, s, d_vin, V32.p, (int64_t)H.ysize);
-      if (nAb)
-        hipLaunchKernelGGL(k_stage_a_big<float>, dim3(nAb), dim3(256), 0, s, tilesAb.p, nAb, L32.p, V32.p, T32.p);
+      if (nAb) launch_a_big<float>(*this, L32.p, V32.p, T32.p, s);
       if (nA) {
         if (H.wave_edge == 16)
           hipLaunchKernelGGL((k_stage_a<float, 16>), dim3(grid_for(nA)), dim3(256), 0, s, tilesA.p, nA, L32.p, V32.p,
@@ -772,12 +978,7 @@ void DevPlan::launch_stage(int stage, const double* d_vin, double* d_vout, hipSt
                              combTerms.p, T32.p, U32.p);
         src = U32.p;
       }
-      if (nCb && H.explicit_u)
-        hipLaunchKernelGGL((k_stage_c_big<float, double, true>), dim3(nCb), dim3(256), 0, s, tilesCb.p, nCb,
-                           chunksC.p, termsC.p, src, R32.p, d_vout);
-      else if (nCb)
-        hipLaunchKernelGGL((k_stage_c_big<float, double, false>), dim3(nCb), dim3(256), 0, s, tilesCb.p, nCb,
-                           chunksC.p, termsC.p, src, R32.p, d_vout);
+      if (nCb) launch_c_big<float>(*this, src, R32.p, d_vout, s);
       if (nC && H.wave_edge == 16)
         hipLaunchKernelGGL((k_stage_c<float, double, 16>), dim3(nC), dim3(256), 0, s, tilesC.p, nC, chunksC.p,
                            termsC.p, src, R32.p, d_vout);

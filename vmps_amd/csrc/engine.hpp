@@ -137,8 +137,11 @@ struct DevPlan {
   // work lists
   DevBuf<TileA> tilesA;
   DevBuf<TileC> tilesC;
-  DevBuf<TileA> tilesAb;  // LDS-staged 128 x 128 tiles (H.big_min64)
+  DevBuf<TileA> tilesAb;  // LDS-staged workgroup tiles (H.big_min64)
   DevBuf<TileC> tilesCb;
+  DevBuf<BigItemC> itemsCb;  // stage C: work items over those tiles, split tiles' reductions
+  DevBuf<BigRedC> redsCb;
+  DevBuf<double> partCb;     // and partial sums (FP64, or FP32 in the lower half)
   DevBuf<ChunkC> chunksC;
   DevBuf<TermC> termsC;
   DevBuf<int64_t> seg_off;

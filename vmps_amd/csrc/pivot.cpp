@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <stdexcept>
 #include <unordered_map>
 #include <unordered_set>
@@ -613,7 +614,7 @@ void make_tiles(const HostPlan& H, int edge, const std::vector<std::pair<int32_t
 
 }  // namespace
 
-std::vector<int64_t> xcd_order(const std::vector<int64_t>& group, const std::vector<int64_t>& cost, int per) {
+std::vector<std::vector<int64_t>> xcd_queues(const std::vector<int64_t>& group, const std::vector<int64_t>& cost) {
   const size_t n = group.size();
   // supertiles in order of first appearance, with their items in list order
   std::unordered_map<int64_t, size_t> gid;
@@ -640,6 +641,11 @@ std::vector<int64_t> xcd_order(const std::vector<int64_t>& group, const std::vec
     queue[x].insert(queue[x].end(), items[g].begin(), items[g].end());
     load[x] += gcost[g];
   }
+  return queue;
+}
+
+std::vector<int64_t> xcd_order(const std::vector<int64_t>& group, const std::vector<int64_t>& cost, int per) {
+  const std::vector<std::vector<int64_t>> queue = xcd_queues(group, cost);
   size_t len = 0;
   for (auto& q : queue) len = std::max(len, q.size());
   len = (len + per - 1) / per * per;
@@ -702,6 +708,99 @@ void order_for_xcds(std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks
   tiles.swap(out);
 }
 
+// Launch order of per-XCD queues: queue x's item k is workgroup k kXcdCount + x.
+template <class T>
+void interleave_queues(const std::vector<std::vector<T>>& queue, const T& padding, std::vector<T>& out) {
+  size_t len = 0;
+  for (const auto& q : queue) len = std::max(len, q.size());
+  out.clear();
+  for (size_t k = 0; k < len; ++k)
+    for (const auto& q : queue) out.push_back(k < q.size() ? q[k] : padding);
+}
+
+// Work items of the LDS-staged stage C tiles.  A tile's K loop runs over all
+// chunks of its output block (1300 steps on C60 at M = 4096), so with one item
+// per tile the last round of workgroups is nearly empty: the CUs were busy 81%
+// of the stage.  The tiles are dealt to the XCDs as supertiles, and the tiles
+// of a supertile are cut along K into the same parts, which run side by side
+// and share operand panels in the XCD's L2 (equal parts per workgroup that
+// ignored the supertiles took 22 ms instead of 12).  Parts get smaller towards
+// the end of a queue: half, then a quarter, then a twelfth of the work that one
+// of the workgroups resident at once has in all.
+void build_big_items(HostPlan& H) {
+  constexpr int64_t kStep = 16, kCu = 256, kMinSteps = 16;
+  const int e = H.big_edge, u = e / 32;
+  H.itemsC_b.clear();
+  H.redsC_b.clear();
+  H.slotsC_b = 0;
+  const size_t n = H.tilesC_b.size();
+  std::vector<int64_t> steps(n, 0), unit(n, 0);
+  for (size_t i = 0; i < n; ++i) {
+    const TileC& t = H.tilesC_b[i];
+    for (int32_t c = t.chunk_begin; c < t.chunk_end; ++c) steps[i] += (H.chunksC[c].K + kStep - 1) / kStep;
+    // a step's MFMAs in 32 x 32 units, plus its barrier and staging
+    unit[i] = std::min<int64_t>(u, (t.M - t.mt * e + 31) / 32) * std::min<int64_t>(u, (t.N - t.nt * e + 31) / 32) + 1;
+  }
+  // supertiles of 4 x 4 tiles, or fewer while the XCDs would have under 16 each
+  std::vector<std::vector<int64_t>> super;
+  for (int edge = 4;; edge /= 2) {
+    super.clear();
+    std::map<std::array<int64_t, 3>, size_t> id;
+    for (size_t i = 0; i < n; ++i) {
+      const TileC& t = H.tilesC_b[i];
+      auto it = id.emplace(std::array<int64_t, 3>{t.c_off, t.mt / edge, t.nt / edge}, super.size());
+      if (it.second) super.emplace_back();
+      super[it.first->second].push_back((int64_t)i);
+    }
+    if (edge == 1 || super.size() >= 16 * kXcdCount) break;
+  }
+  std::vector<int64_t> group(super.size()), cost(super.size(), 0);
+  for (size_t g = 0; g < super.size(); ++g) {
+    group[g] = (int64_t)g;
+    for (int64_t i : super[g]) cost[g] += steps[i] * unit[i];
+  }
+  const double resident = (double)(kCu / kXcdCount) * (e == 64 ? 3 : 2);
+  std::vector<std::vector<BigItemC>> items(kXcdCount);
+  const std::vector<std::vector<int64_t>> queue = xcd_queues(group, cost);
+  for (int x = 0; x < kXcdCount; ++x) {
+    double total = 0, done = 0;
+    for (int64_t g : queue[x]) total += (double)cost[g];
+    for (int64_t g : queue[x]) {
+      const double f = total > 0 ? done / total : 0.0;
+      const double most = std::max(1.0, total / resident * (f < 0.5 ? 0.5 : f < 0.8 ? 0.25 : 1.0 / 12));
+      int64_t S = 1, fewest = std::numeric_limits<int64_t>::max();
+      for (int64_t i : super[g]) {
+        S = std::max(S, (int64_t)std::ceil((double)(steps[i] * unit[i]) / most));
+        fewest = std::min(fewest, steps[i]);
+      }
+      S = std::max<int64_t>(1, std::min(S, fewest / kMinSteps));
+      std::vector<std::array<int64_t, 2>> at;  // (chunk, step within it) where the next part of a tile starts
+      for (int64_t i : super[g]) at.push_back({H.tilesC_b[i].chunk_begin, 0});
+      for (int64_t p = 0; p < S; ++p)
+        for (size_t j = 0; j < super[g].size(); ++j) {
+          const int64_t i = super[g][j];
+          const TileC& t = H.tilesC_b[i];
+          const int64_t k = steps[i] * (p + 1) / S - steps[i] * p / S;
+          int64_t &c = at[j][0], &st = at[j][1];
+          items[x].push_back({(int32_t)i, (int32_t)c, (int32_t)st, (int32_t)k,
+                              S > 1 ? H.slotsC_b + (int64_t)j * S + p : -1});
+          for (st += k; c < t.chunk_end; ++c) {
+            const int64_t nc = (H.chunksC[c].K + kStep - 1) / kStep;
+            if (st < nc) break;
+            st -= nc;
+          }
+        }
+      if (S > 1)
+        for (size_t j = 0; j < super[g].size(); ++j) {
+          H.redsC_b.push_back({H.slotsC_b, (int32_t)super[g][j], (int32_t)S});
+          H.slotsC_b += S;
+        }
+      done += (double)cost[g];
+    }
+  }
+  interleave_queues(items, BigItemC{-1, 0, 0, 0, -1}, H.itemsC_b);
+}
+
 int choose_wave_edge(const HostPlan& H) {
   if (const char* e = std::getenv("VMPS_WAVE_TILE")) {
     const int v = std::atoi(e);
@@ -719,12 +818,24 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
   H.big_min64 = big_min64;
   if (big_min64 > 0) {
     make_tiles(H, edge, H.crange, H.tilesA_w, H.tilesC_w, -big_min64);
-    make_tiles(H, kBigTile, H.crange, H.tilesA_b, H.tilesC_b, big_min64);
+    // 128 x 128 tiles once stage C's blocks of 128 and more give each of the 256 CUs one:
+    // below that the K loops would have to be cut into parts too short for
+    // their partial sums (FP64, 64 against 128 wide, all problems: C60 at
+    // M = 1024 676 / 800 us, U(1) chain at M = 2048 263 / 301 us; C60 at
+    // M = 2048 3.73 / 3.56 ms, at M = 4096 25.3 / 23.7 ms).
+    int64_t tiles128 = 0;
+    for (const GemmProb& pr : H.probC)
+      if (pr.M >= 128 && pr.N >= 128) tiles128 += (int64_t)((pr.M + 127) / 128) * ((pr.N + 127) / 128);
+    H.big_edge = tiles128 >= 256 ? 128 : 64;
+    make_tiles(H, H.big_edge, H.crange, H.tilesA_b, H.tilesC_b, big_min64);
     order_for_xcds(H.tilesA_b);
-    order_for_xcds(H.tilesC_b, H.chunksC);
+    build_big_items(H);
   } else {
     H.tilesA_b.clear();
     H.tilesC_b.clear();
+    H.itemsC_b.clear();
+    H.redsC_b.clear();
+    H.slotsC_b = 0;
     if (edge == kTile) {
       H.tilesA_w = H.tilesA;
       H.tilesC_w = H.tilesC;
@@ -1085,12 +1196,16 @@ void build_plan_tables(const TripleSet& S, HostPlan& H) {
 
   validate_host_plan(H);
   // Pivots with blocks of 256 and more start from the explicit stage B and
-  // the FP64 / FP32 big tiles, which the autotuner picks on every such pivot
-  // measured; the tuner then finds the lists already built for its first
-  // candidate instead of building them a second time.
+  // the FP64 / FP32 LDS-staged tiles for every problem, which the autotuner
+  // picks on every such pivot measured; the tuner then finds the lists already
+  // built for its first candidate instead of building them a second time.
+  // For every problem, since a second launch for the small blocks runs on a
+  // nearly empty chip: with blocks below 128 or 32 on wave tiles the U(1) chain at
+  // M = 2048 took 283 or 281 instead of 263 us, C60 at M = 1024 780 or 709
+  // instead of 676 us.
   if (st.max_block_dim >= 2 * kBigTile) {
     H.explicit_u = true;
-    if (H.big_min64 <= 0) H.big_min64 = kBigTile;
+    if (H.big_min64 <= 0) H.big_min64 = 1;
   }
   build_tiles(H);
   st.n_terms = (int64_t)terms.size();

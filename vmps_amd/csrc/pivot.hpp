@@ -228,6 +228,18 @@ struct TileC {             // Vout(M x N, ld M) tile = sum over chunks U . R
   int16_t mt, nt;
   int32_t pad;
 };
+// LDS-staged FP64 / FP32 tiles of stage C: K steps [step, step + nsteps) of the
+// tile's flattened (chunk, 16-deep K step) sequence, counted from `step` of
+// chunk `chunk`.  slot < 0: the item is the whole tile and writes the output;
+// else it writes partial tile `slot`.
+struct BigItemC {
+  int32_t tile, chunk, step, nsteps;  // tile < 0: padding of the launch order
+  int64_t slot;
+};
+struct BigRedC {           // tile = sum of its nsplit partial tiles from `slot` on
+  int64_t slot;
+  int32_t tile, nsplit;
+};
 struct ChunkC {            // one (U_u, R_r) pair: U_u = sum_j c_j T_j (M x K), R_r (K x N, ld K)
   int64_t r_off;
   int32_t K;
@@ -370,11 +382,15 @@ struct HostPlan {
   // kBigTile tiles (big_min <= 0: none do)
   int big_min = kBigMin;
   // FP64 / FP32: problems with both dimensions >= big_min64 take the
-  // LDS-staged kBigTile tiles tilesA_b / tilesC_b and are absent from the wave
-  // lists (0: none do, the default)
+  // LDS-staged tiles tilesA_b / tilesC_b and are absent from the wave
+  // lists (0: none do)
   int big_min64 = 0;
   std::vector<TileA> tilesA_b;
   std::vector<TileC> tilesC_b;
+  int big_edge = 128;                 // their edge, 64 or 128
+  std::vector<BigItemC> itemsC_b;     // stage C work items over tilesC_b
+  std::vector<BigRedC> redsC_b;       // tiles split over several items
+  int64_t slotsC_b = 0;               // partial tiles of those
   // stage B: false = fused into stage C's operand load (U never stored);
   // true = U formed by its own kernel (comb_tasks / comb_terms) and stage C's
   // chunks read U with one unit-weight term each (termsC t_off = U offsets)
@@ -432,6 +448,8 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64);
 // Returns item indices in launch order; -1 marks padding slots, filled with
 // empty items, that keep later items on their XCD.
 constexpr int kXcdCount = 8;
+// the XCD queues themselves (item indices, in order)
+std::vector<std::vector<int64_t>> xcd_queues(const std::vector<int64_t>& group, const std::vector<int64_t>& cost);
 std::vector<int64_t> xcd_order(const std::vector<int64_t>& group, const std::vector<int64_t>& cost, int per = 1);
 // wave tile lists at least this long are grouped per XCD (set_wave_edge)
 constexpr size_t kXcdMinTilesA = 2048, kXcdMinTilesC = 512;
