@@ -112,3 +112,26 @@ def test_batch64_bf16x3_hxv_matches_oracle_subset():
         ref = pivots.oracle_hxv(lib, h, vin[i], 16)
         lib.oracle_pivot2_destroy(h)
         assert np.linalg.norm(out[i] - ref) <= 5e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("iters", [3, 18, 37])
+def test_batch_gram_schmidt_chunks(iters):
+    """A pivot of a few elements next to one long enough for chunks of 512
+    elements, at iteration counts inside, at and past a group of 16 basis rows:
+    every pivot's Ritz value equals that of its own single-plan solve (which sums
+    in another order: 1e-11 relative, as above).  The small pivot's Krylov space
+    ends before the large one's solve does."""
+    rng = np.random.default_rng(31)
+    heis = models.heisenberg_u1_mpo()
+    pds = [synth.make_pivot(heis, heis, synth.heisenberg_bond(n, M), synth.heisenberg_bond(n + 2, M), rng,
+                            hermitian=True) for n, M in ((5, 8), (20, 1400), (9, 31))]
+    B = PivotBatch(pds)
+    v0 = np.random.default_rng(32).uniform(-1, 1, B.vsize)
+    opts = dict(max_iter=iters, tol_eigval=0.0, tol_state=0.0)
+    _, rb = lanczos_batch(B, v0=v0, **opts)
+    for i, pd in enumerate(pds):
+        H = PivotMatrix2(pd)
+        _, rs = lanczos(H, v0=B.split(v0)[i], **opts)
+        print("pivot", i, "vsize", pd.vsize, rb[i]["energy"], rs["energy"], flush=True)
+        assert abs(rb[i]["energy"] - rs["energy"]) <= 1e-11 * max(1.0, abs(rs["energy"]))
+        H.close()

@@ -59,7 +59,6 @@ struct BChunk {
 // the concatenated vector of a batch plan, every reduction segmented by pivot.
 struct BatchKrylov {
   static constexpr int kIterBatch = 4;
-  static constexpr int64_t kChunk = 4096;
   int P = 0;
   int64_t n = 0;
   std::vector<int64_t> off;   // pivot p owns [off[p], off[p+1])
@@ -68,15 +67,16 @@ struct BatchKrylov {
   int nc = 0;
   DevBuf<double> Q, w, v, c, gpart, npart, nv, out3, ew, Y, spart, sres, coefa, coefb;
   DevBuf<int> kdev;
-  double* host = nullptr;     // pinned readback of one graph launch's scalars
+  double* host = nullptr;     // pinned readback of two graph launches' scalars
+  hipEvent_t landed[2] = {nullptr, nullptr};  // a slot's readback has landed
   int cap = 0;
   hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
-  hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
+  hipGraphExec_t exec[3][2] = {};  // two instances of each graph
   int graph_gen[3] = {-1, -1, -1};
   void setup(DevPlan& D, const std::vector<int64_t>& offsets);
   void ensure(DevPlan& D, int kmax);
   void enqueue_iteration(DevPlan& D, hipStream_t s, int kofs);
-  hipGraphExec_t ensure_graph(DevPlan& D);
+  hipGraphExec_t ensure_graph(DevPlan& D, int copy);
   void release_graph();
   std::vector<double> seg_dot(DevPlan& D, const double* x, const double* y);
   void piv_axpby(DevPlan& D, const std::vector<double>& a, const double* x, const std::vector<double>& b, double* y);

@@ -37,47 +37,98 @@ __device__ inline double wg_sum_b(double x) {
   return r;
 }
 
-// partial[i * nc + b] = sum over chunk b of ew Q_i w, rows i = 4y .. 4y+3 <= k
+// sum over the 64 lanes in a fixed order, on every lane
+__device__ inline double wave_sum_b(double x) {
+  for (int m = 32; m > 0; m >>= 1) x += __shfl_xor(x, m);
+  return x;
+}
+
+// The Gram-Schmidt kernels of a batch of small pivots wait for memory, not for
+// bandwidth: 8 pivots of M <= 256 are 69k elements, and with chunks of 4096
+// elements 21 workgroups walked the basis row by row (k_bsub 235 us, k_bdot_rows
+// 24 us on average over 120 iterations).  Hence short chunks
+// (BatchKrylov::setup), one wave per four rows with 16 basis loads in flight per
+// lane in the dots, and 16 rows in flight per element in the subtraction
+// (9.5 us and 9.0 us).
+
+// partial[i * nc + b] = sum over chunk b of ew Q_i w for the rows i <= k of wave
+// threadIdx.x / 64: i = 16 y + 4 wave .. + 3
 __global__ __launch_bounds__(256) void k_bdot_rows(const int* __restrict__ kdev, int kofs,
                                                    const double* __restrict__ Q, int64_t n,
                                                    const double* __restrict__ w, const double* __restrict__ ew,
                                                    const BChunk* __restrict__ ch, int nc,
                                                    double* __restrict__ partial) {
   const int k = *kdev + kofs;
-  const int i0 = 4 * blockIdx.y;
-  if (i0 > k) return;  // workgroup-uniform
-  __shared__ double ws[4][4];
-  const int nr = min(4, k + 1 - i0);
+  const int i0 = 16 * blockIdx.y + 4 * (threadIdx.x >> 6);
+  if (i0 > k) return;  // wave-uniform; the kernel has no barrier
+  const int lane = threadIdx.x & 63;
   const BChunk c = ch[blockIdx.x];
+  const double* __restrict__ q[4];  // rows past k read row k again (their sums are not stored)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) q[r] = Q + (int64_t)min(i0 + r, k) * n + c.start;
+  w += c.start;
+  ew += c.start;
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int64_t e = c.start + threadIdx.x; e < c.start + c.len; e += 256) {
+  int e = lane;
+  for (; e + 192 < c.len; e += 256) {
+    double we[4], x[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      we[u] = w[e + 64 * u] * ew[e + 64 * u];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[u][r] = q[r][e + 64 * u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] += x[u][r] * we[u];
+  }
+  for (; e < c.len; e += 64) {
     const double we = w[e] * ew[e];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (r < nr) acc[r] += Q[(int64_t)(i0 + r) * n + e] * we;
+    for (int r = 0; r < 4; ++r) acc[r] += q[r][e] * we;
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    double x = acc[r];
-    for (int m = 32; m > 0; m >>= 1) x += __shfl_xor(x, m);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6][r] = x;
-  }
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (t < nr) partial[(int64_t)(i0 + t) * nc + blockIdx.x] = (ws[0][t] + ws[1][t]) + (ws[2][t] + ws[3][t]);
+  for (int r = 0; r < 4; ++r) acc[r] = wave_sum_b(acc[r]);
+  if (lane < 4 && i0 + lane <= k)
+    partial[(int64_t)(i0 + lane) * nc + blockIdx.x] = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
 }
 
-// c[i * P + p] = sum of partial[i * nc + b] over the chunks b of pivot p;
-// workgroup (p, i), rows past k exit
+// c[i * P + p] = sum of partial[i * nc + b] over the chunks b of pivot p; one
+// wave per row i = 4 y + threadIdx.x / 64
 __global__ __launch_bounds__(256) void k_bdot_final(const int* __restrict__ kdev, int kofs,
                                                     const double* __restrict__ partial, int nc,
                                                     const int32_t* __restrict__ cb, int P, double* __restrict__ c) {
-  const int p = blockIdx.x, i = blockIdx.y;
-  if (i > *kdev + kofs) return;  // workgroup-uniform
+  const int p = blockIdx.x, i = 4 * blockIdx.y + (threadIdx.x >> 6);
+  if (i > *kdev + kofs) return;  // wave-uniform; the kernel has no barrier
+  const int lane = threadIdx.x & 63;
   double acc = 0.0;
-  for (int b = cb[p] + threadIdx.x; b < cb[p + 1]; b += 256) acc += partial[(int64_t)i * nc + b];
-  acc = wg_sum_b(acc);
-  if (threadIdx.x == 0) c[(int64_t)i * P + p] = acc;
+#pragma unroll 4
+  for (int b = cb[p] + lane; b < cb[p + 1]; b += 64) acc += partial[(int64_t)i * nc + b];
+  acc = wave_sum_b(acc);
+  if (lane == 0) c[(int64_t)i * P + p] = acc;
+}
+
+// sum_{i<m} c[i] Q_i[e], added in order of i, with 16 basis loads in flight
+__device__ inline double rows_at(const double* __restrict__ Q, int64_t n, const double* c, int m, int64_t e) {
+  double s = 0.0;
+  int i = 0;
+  for (; i + 16 <= m; i += 16) {
+    double q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = Q[(int64_t)(i + u) * n + e];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += c[i + u] * q[u];
+  }
+  if (i < m) {  // rows past m read row m - 1 again, with weight 0
+    double q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = Q[(int64_t)min(i + u, m - 1) * n + e];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (i + u < m) s += c[i + u] * q[u];
+  }
+  return s;
 }
 
 // w -= sum_{i<=k} c[i * P + p] Q_i over every chunk (p its pivot); with
@@ -96,9 +147,7 @@ __global__ __launch_bounds__(256) void k_bsub(const double* __restrict__ Q, int6
     __syncthreads();
     double nrm = 0.0;
     for (int64_t e = cbk.start + threadIdx.x; e < cbk.start + cbk.len; e += 256) {
-      double s = 0.0;
-      for (int i = 0; i <= k; ++i) s += cs[i] * Q[(int64_t)i * n + e];
-      const double y = w[e] - s;
+      const double y = w[e] - rows_at(Q, n, cs, k + 1, e);
       w[e] = y;
       nrm += ew[e] * y * y;
     }
@@ -191,9 +240,7 @@ __global__ __launch_bounds__(256) void k_bcombination(const double* __restrict__
     const BChunk cbk = ch[b];
     const double* __restrict__ yc = Y + (int64_t)cbk.piv * ldy;
     for (int64_t e = cbk.start + threadIdx.x; e < cbk.start + cbk.len; e += 256) {
-      double s = 0.0;
-      for (int i = 0; i < kuse; ++i) s += yc[i] * Q[(int64_t)i * n + e];
-      y[e] = s;
+      y[e] = rows_at(Q, n, yc, kuse, e);
     }
   }
 }
@@ -215,9 +262,11 @@ void BatchKrylov::setup(DevPlan& D, const std::vector<int64_t>& offsets) {
   off = offsets;
   std::vector<BChunk> hc;
   std::vector<int32_t> hb(1, 0);
+  // about 2048 chunks (8 workgroups per CU), of 256 to 4096 elements
+  const int64_t chunk = std::max<int64_t>(256, std::min<int64_t>(4096, (n / 2048 + 255) / 256 * 256));
   for (int p = 0; p < P; ++p) {
-    for (int64_t s = off[p]; s < off[p + 1]; s += kChunk)
-      hc.push_back({s, (int32_t)std::min<int64_t>(kChunk, off[p + 1] - s), p});
+    for (int64_t s = off[p]; s < off[p + 1]; s += chunk)
+      hc.push_back({s, (int32_t)std::min<int64_t>(chunk, off[p + 1] - s), p});
     hb.push_back((int32_t)hc.size());
   }
   nc = (int)hc.size();
@@ -253,19 +302,21 @@ void BatchKrylov::ensure(DevPlan& D, int kmax) {
   Y.alloc((size_t)P * (need + 1));
   if (host) (void)hipHostFree(host);
   host = nullptr;
-  VMPS_HIP_CHECK(hipHostMalloc((void**)&host, 4 * (size_t)kIterBatch * P * sizeof(double), hipHostMallocDefault));
+  VMPS_HIP_CHECK(hipHostMalloc((void**)&host, 8 * (size_t)kIterBatch * P * sizeof(double), hipHostMallocDefault));
+  for (auto& e : landed)
+    if (!e) VMPS_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   VMPS_HIP_CHECK(hipStreamSynchronize(D.stream));
   cap = need;
 }
 
 void BatchKrylov::enqueue_iteration(DevPlan& D, hipStream_t s, int kofs) {
-  const unsigned gy = (unsigned)((cap + 3) / 4);
+  const unsigned gy = (unsigned)((cap + 15) / 16), gf = (unsigned)((cap + 3) / 4);
   double* c1 = c.p;
   double* c2 = c.p + (size_t)(cap + 1) * P;
   auto pass = [&](double* c_out, double* norm_part) {
     hipLaunchKernelGGL(k_bdot_rows, dim3(nc, gy), dim3(256), 0, s, kdev.p, kofs, Q.p, n, w.p, ew.p, ch.p, nc,
                        gpart.p);
-    hipLaunchKernelGGL(k_bdot_final, dim3(P, cap), dim3(256), 0, s, kdev.p, kofs, gpart.p, nc, cb.p, P, c_out);
+    hipLaunchKernelGGL(k_bdot_final, dim3(P, gf), dim3(256), 0, s, kdev.p, kofs, gpart.p, nc, cb.p, P, c_out);
     hipLaunchKernelGGL(k_bsub, dim3(bgrid(nc)), dim3(256), 0, s, Q.p, n, c_out, P, kdev.p, kofs, ch.p, nc, w.p,
                        ew.p, norm_part);
   };
@@ -280,20 +331,27 @@ void BatchKrylov::enqueue_iteration(DevPlan& D, hipStream_t s, int kofs) {
 
 void BatchKrylov::release_graph() {
   for (int i = 0; i < 3; ++i) {
-    if (exec[i]) (void)hipGraphExecDestroy(exec[i]);
+    for (auto& e : exec[i]) {
+      if (e) (void)hipGraphExecDestroy(e);
+      e = nullptr;
+    }
     if (graph[i]) (void)hipGraphDestroy(graph[i]);
-    exec[i] = nullptr;
     graph[i] = nullptr;
     graph_gen[i] = -1;
   }
 }
 
-hipGraphExec_t BatchKrylov::ensure_graph(DevPlan& D) {
+hipGraphExec_t BatchKrylov::ensure_graph(DevPlan& D, int copy) {
   const int p = (int)D.prec;
-  if (exec[p] && graph_gen[p] == D.gen) return exec[p];
-  if (exec[p]) (void)hipGraphExecDestroy(exec[p]);
+  if (graph[p] && graph_gen[p] == D.gen) {
+    if (!exec[p][copy]) VMPS_HIP_CHECK(hipGraphInstantiate(&exec[p][copy], graph[p], nullptr, nullptr, 0));
+    return exec[p][copy];
+  }
+  for (auto& e : exec[p]) {
+    if (e) (void)hipGraphExecDestroy(e);
+    e = nullptr;
+  }
   if (graph[p]) (void)hipGraphDestroy(graph[p]);
-  exec[p] = nullptr;
   graph[p] = nullptr;
   hipStream_t s = D.stream;
   VMPS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -307,14 +365,16 @@ hipGraphExec_t BatchKrylov::ensure_graph(DevPlan& D) {
     throw;
   }
   VMPS_HIP_CHECK(hipStreamEndCapture(s, &graph[p]));
-  VMPS_HIP_CHECK(hipGraphInstantiate(&exec[p], graph[p], nullptr, nullptr, 0));
   graph_gen[p] = D.gen;
-  return exec[p];
+  VMPS_HIP_CHECK(hipGraphInstantiate(&exec[p][copy], graph[p], nullptr, nullptr, 0));
+  return exec[p][copy];
 }
 
 BatchKrylov::~BatchKrylov() {
   release_graph();
   if (host) (void)hipHostFree(host);
+  for (auto& e : landed)
+    if (e) (void)hipEventDestroy(e);
 }
 
 // per-pivot weighted dots <x, y> of the batch vectors (synchronous)
@@ -353,7 +413,7 @@ std::vector<LanczosResult> lanczos_solve_batch(DevPlan& D, BatchKrylov& K, doubl
   try {
     D.ensure_precision_buffers();
     K.ensure(D, kmax);
-    hipGraphExec_t iteration = o.graph ? K.ensure_graph(D) : nullptr;
+    hipGraphExec_t iteration[2] = {o.graph ? K.ensure_graph(D, 0) : nullptr, o.graph ? K.ensure_graph(D, 1) : nullptr};
     // q0 = v / ||v|| per pivot, into the basis and the HxV input
     std::vector<double> nrm = K.seg_dot(D, d_v, d_v), a(P), z(P, 0.0);
     for (int p = 0; p < P; ++p) {
@@ -378,23 +438,50 @@ std::vector<LanczosResult> lanczos_solve_batch(DevPlan& D, BatchKrylov& K, doubl
         if (!done[p]) return false;
       return true;
     };
+    // The host's tridiagonal solves of a batch of iterations (P pivots, one
+    // after the other) take longer than the device's part: while the last batch
+    // read left some pivot's residual estimate or eigenvalue change at least
+    // 100x above its tolerance, the next batch is queued before the host turns
+    // to the current one (8 pivots of M <= 256, 120 iterations: 17.5 -> 11.6 ms).
+    // Two instances of the graph and two readback slots alternate.
+    constexpr int B = BatchKrylov::kIterBatch;
+    const size_t slot_elems = 4 * (size_t)B * P;
+    bool far = false;
+    int kq = 0, inflight = 0, head = 0;  // next iteration to queue, batches queued and not read, oldest one's slot
+    auto queue_batch = [&]() {
+      const int slot = (head + inflight) & 1;
+      VMPS_HIP_CHECK(hipGraphLaunch(iteration[(kq / B) & 1], s));
+      VMPS_HIP_CHECK(hipMemcpyAsync(K.host + slot * slot_elems, K.out3.p + 4 * (size_t)kq * P,
+                                    slot_elems * sizeof(double), hipMemcpyDeviceToHost, s));
+      VMPS_HIP_CHECK(hipEventRecord(K.landed[slot], s));
+      kq += B;
+      ++inflight;
+      hxv += B;
+    };
     while (k < kmax && !all_done()) {
       int nb = 1;
-      if (iteration) {
-        VMPS_HIP_CHECK(hipGraphLaunch(iteration, s));
-        nb = BatchKrylov::kIterBatch;
+      const double* hs = K.host;
+      if (iteration[0]) {
+        if (inflight == 0) queue_batch();
+        if (far && inflight == 1 && kq < kmax) queue_batch();
+        VMPS_HIP_CHECK(hipEventSynchronize(K.landed[head]));
+        hs = K.host + head * slot_elems;
+        head ^= 1;
+        --inflight;
+        nb = B;
       } else {
         K.enqueue_iteration(D, s, 0);
         hipLaunchKernelGGL(k_badd_int, dim3(1), dim3(64), 0, s, K.kdev.p, 1);
+        VMPS_HIP_CHECK(hipMemcpyAsync(K.host, K.out3.p + 4 * (size_t)k * P, 4 * (size_t)P * sizeof(double),
+                                      hipMemcpyDeviceToHost, s));
+        VMPS_HIP_CHECK(hipStreamSynchronize(s));
+        ++hxv;
       }
-      hxv += nb;
-      VMPS_HIP_CHECK(hipMemcpyAsync(K.host, K.out3.p + 4 * (size_t)k * P, 4 * (size_t)nb * P * sizeof(double),
-                                    hipMemcpyDeviceToHost, s));
-      VMPS_HIP_CHECK(hipStreamSynchronize(s));
       for (int j = 0; j < nb && k < kmax; ++j, ++k) {
+        far = false;
         for (int p = 0; p < P; ++p) {
           if (done[p]) continue;
-          const double* h3 = K.host + 4 * ((size_t)j * P + p);
+          const double* h3 = hs + 4 * ((size_t)j * P + p);
           const double a_k = h3[0] + h3[1];
           const double b_k = std::sqrt(std::max(0.0, h3[2]));
           alpha[p].push_back(a_k);
@@ -408,10 +495,14 @@ std::vector<LanczosResult> lanczos_solve_batch(DevPlan& D, BatchKrylov& K, doubl
                             rest < o.tol_state)) {
             done[p] = 1;
             res[p].converged = true;
+          } else if (k > 0 && (std::fabs(E[p] - Eprev[p]) > 100.0 * o.tol_eigval || rest > 100.0 * o.tol_state)) {
+            far = true;
           }
         }
       }
     }
+    // a batch queued past convergence runs before the work below (stream order)
+    // and only extends the basis
     // Ritz vectors: pivot p combines its own first iterations[p] basis rows
     const int ldy = K.cap + 1;
     std::vector<double> Yh((size_t)P * ldy, 0.0);
