@@ -166,11 +166,21 @@ def test_lds_tiles_at_block_edges(edge_case, precision, tol, big_min64, xu):
     assert _rel(HxV(H, v), ref) <= tol
 
 
+@pytest.mark.parametrize("big_min,xu", [(1, 1), (1, 0), (33, 1), (0, 1)])
+def test_bf16x3_tiles_at_block_edges(edge_case, big_min, xu):
+    pd, v, ref = edge_case
+    print("split-BF16 tiles at edges", big_min, xu, flush=True)
+    H = PivotMatrix2(pd, precision="bf16x3")
+    H.set_tiles(big_min=big_min, explicit_u=xu)
+    assert _rel(HxV(H, v), ref) <= BF16X3_RTOL
+
+
 @pytest.mark.parametrize("M,nleft", [(640, 29), (2047, 30)])
 def test_lds_tiles_split_k(M, nleft):
     """Stage C tiles cut along K, in 64-wide (M = 640) and 128-wide (M = 2047)
     tiles, against the wave tiles: both sum a few thousand products per element
-    in FP64, so they agree to 1e-13 of the result's norm."""
+    in FP64, so they agree to 1e-13 of the result's norm.  The split-BF16 tiles
+    against that result."""
     from vmps_amd import models
     W = models.heisenberg_su2_lr_mpo(synth.lr_couplings(3, np.random.default_rng(1)))
     pd = synth.make_pivot(W, W, synth.heisenberg_su2_bond(nleft, M), synth.heisenberg_su2_bond(nleft + 2, M),
@@ -184,3 +194,8 @@ def test_lds_tiles_split_k(M, nleft):
     out = HxV(H, v)
     assert _rel(out, ref) <= 1e-13
     assert np.array_equal(HxV(H, v), out)  # a fixed order of summation
+    H.set_precision("bf16x3")
+    H.set_tiles(big_min=1, explicit_u=1)
+    out = HxV(H, v)
+    assert _rel(out, ref) <= BF16X3_RTOL
+    assert np.array_equal(HxV(H, v), out)

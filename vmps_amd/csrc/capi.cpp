@@ -732,13 +732,17 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
     return (double)ms / iters;
   };
   TileChoice pick{D.H.wave_edge, D.H.big_min, D.H.big_min64, D.H.explicit_u};
-  // Pivots with blocks of 256 and more keep the FP64 / FP32 LDS-staged tiles
-  // with the explicit stage B, which their plans start from: wave tiles take
-  // 1.3 to 2.5 times as long (C60 at M = 4096: 58 against 24 ms; U(1) chain at
-  // M = 2048: 339 against 263 us), the fused stage B 1.1 to 1.3 times.
-  const bool large = D.H.stats.max_block_dim >= 2 * vmps::kBigTile && D.prec != VMPS_PREC_BF16X3;
-  if (large && pick.big_min64 <= 0) pick.big_min64 = 1;
-  if (large) pick.explicit_u = true;
+  // Pivots with blocks of 256 and more keep the LDS-staged tiles with the
+  // explicit stage B, which their plans start from, and nothing is left to
+  // time: wave tiles take 1.3 to 2.5 times as long (FP64: C60 at M = 4096 58
+  // against 24 ms, U(1) chain at M = 2048 339 against 263 us; split-BF16: 174
+  // against 96 us there), the fused stage B 1.1 to 1.4 times.
+  const bool large = D.H.stats.max_block_dim >= 2 * vmps::kBigTile;
+  if (large) {
+    pick.explicit_u = true;
+    int& threshold = D.prec == VMPS_PREC_BF16X3 ? pick.big_min : pick.big_min64;
+    if (threshold <= 0) threshold = 1;
+  }
   double best = measure(pick);
   int tried = 1;
   auto consider = [&](TileChoice c) {
@@ -752,7 +756,7 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
       pick = c;
     }
   };
-  if (D.prec == VMPS_PREC_BF16X3) {
+  if (!large && D.prec == VMPS_PREC_BF16X3) {
     const TileChoice base = pick;
     for (int b : {vmps::kBigMin, 2 * vmps::kBigMin, 0}) {
       TileChoice c = base;
@@ -770,12 +774,12 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
     c.explicit_u = true;
     consider(c);
   }
-  for (bool xu : {false, true}) {
-    if (large && !xu) continue;
-    TileChoice c = pick;
-    c.explicit_u = xu;
-    consider(c);
-  }
+  if (!large)
+    for (bool xu : {false, true}) {
+      TileChoice c = pick;
+      c.explicit_u = xu;
+      consider(c);
+    }
   D.retile(pick.wave_edge, pick.big_min, pick.big_min64, pick.explicit_u);
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);

@@ -1,5 +1,6 @@
-// Explicit stage B kernel shared by the FP64 / FP32 and split-BF16 paths:
-// U_u = sum_j c_j T_j elementwise over blocks of equal shape and layout.
+// Explicit stage B kernel of the FP64 / FP32 path (U_u = sum_j c_j T_j
+// elementwise over blocks of equal shape and layout), and the reduction of the
+// stage C tiles cut along K, shared with the split-BF16 path.
 #pragma once
 #include "pivot.hpp"
 #include "wave.hpp"
@@ -82,6 +83,26 @@ __global__ __launch_bounds__(256) void k_combine(const CombTask* __restrict__ ta
       for (int q = 0; q < W; ++q)
         if (e + q < t.n) dst[e + q] = acc[v][q];
     }
+  }
+}
+
+// Vout tile = sum over its split partials, in slot order; one workgroup per
+// quarter of a tile's columns.
+template <class T, class OutT, int BT>
+__global__ __launch_bounds__(256) void k_reduce_big(const TileC* __restrict__ tiles, const BigRedC* __restrict__ reds,
+                                                    const T* __restrict__ partial, OutT* __restrict__ Vout) {
+  const BigRedC r = reds[blockIdx.x / 4];
+  const TileC t = tiles[r.tile];
+  const int i = t.mt * BT + threadIdx.x % BT;
+  if (i >= t.M) return;
+  const int c0 = (int)(blockIdx.x % 4) * (BT / 4) + threadIdx.x / BT;
+  for (int c = c0; c < (int)(blockIdx.x % 4 + 1) * (BT / 4); c += 256 / BT) {
+    const int j = t.nt * BT + c;
+    if (j >= t.N) return;
+    const T* p = partial + r.slot * (int64_t)(BT * BT) + c * BT + threadIdx.x % BT;
+    T acc = p[0];
+    for (int q = 1; q < r.nsplit; ++q) acc += p[(int64_t)q * (BT * BT)];
+    Vout[t.c_off + (int64_t)j * t.M + i] = (OutT)acc;
   }
 }
 

@@ -639,26 +639,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
 }
 
-// Vout tile = sum over its split partials, in slot order; one workgroup per
-// quarter of a tile's columns.
-template <class T, class OutT, int BT>
-__global__ __launch_bounds__(256) void k_reduce_big(const TileC* __restrict__ tiles, const BigRedC* __restrict__ reds,
-                                                    const T* __restrict__ partial, OutT* __restrict__ Vout) {
-  const BigRedC r = reds[blockIdx.x / 4];
-  const TileC t = tiles[r.tile];
-  const int i = t.mt * BT + threadIdx.x % BT;
-  if (i >= t.M) return;
-  const int c0 = (int)(blockIdx.x % 4) * (BT / 4) + threadIdx.x / BT;
-  for (int c = c0; c < (int)(blockIdx.x % 4 + 1) * (BT / 4); c += 256 / BT) {
-    const int j = t.nt * BT + c;
-    if (j >= t.N) return;
-    const T* p = partial + r.slot * (int64_t)(BT * BT) + c * BT + threadIdx.x % BT;
-    T acc = p[0];
-    for (int q = 1; q < r.nsplit; ++q) acc += p[(int64_t)q * (BT * BT)];
-    Vout[t.c_off + (int64_t)j * t.M + i] = (OutT)acc;
-  }
-}
-
 // Weighted dot product, pass 1: workgroup b reduces segments [b*spb, (b+1)*spb).
 __global__ __launch_bounds__(256) void k_dot_partial(const int64_t* __restrict__ seg_off, const int32_t* __restrict__ seg_len,
                                                      const double* __restrict__ seg_w, int nseg, int spb,

@@ -120,17 +120,16 @@ struct DevPlan {
   DevBuf<TermC> combTerms;
 
   // split-BF16 x3 operands, intermediates and work lists
-  DevBuf<uint16_t> Lhi, Llo, Rhi, Rlo, Vhi, Vlo;
+  DevBuf<uint16_t> Ls, Rs, Vs, Us;  // groups of [8 hi | 8 lo]; Us: explicit stage B
   DevBuf<float> Tp;
   DevBuf<TileA16> bfA, bfAbig;
   DevBuf<TileC> bfCsmall, bfCbig;
-  DevBuf<int32_t> wTile, wBegin, wEnd, rTile, rNs;  // split-K work items / reductions
-  DevBuf<int64_t> wSlot, rSlot;
+  DevBuf<BigItemC> itemsC16;  // work items over bfCbig, and the tiles in several of them
+  DevBuf<BigRedC> redsC16;
   DevBuf<float> Cpart;                              // FP32 partial tiles
   DevBuf<ChunkC16> bfC;
   DevBuf<TermC16> bfT;
   DevBuf<VConv> vconv;
-  DevBuf<float> Up;                     // explicit stage B: padded FP32 U
   DevBuf<CombTask> bfCombTasks;
   DevBuf<TermC16> bfCombTerms;
 

@@ -3,9 +3,14 @@
 // Every FP64 operand x is carried as hi = bf16(x), lo = bf16(x - hi); a
 // product a.b is formed as a_hi.b_hi + a_hi.b_lo + a_lo.b_hi by three
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation (relative error ~1e-5).
-// Operands are k-contiguous with k padded to a multiple of 8 (one aligned
-// 16-byte load = one MFMA lane's 8 k values; the zero padding ends K):
-//   L^T (row-major M x Kp), V and R (column-major Kp x N), T (row-major M x Np).
+// Operands are k-contiguous with k padded to a multiple of 8 and stored in groups
+// of [8 hi | 8 lo] (32 bytes; the zero padding ends K): an MFMA lane's 8 k values
+// are one aligned 16-byte load for hi and the next one for lo, and a 32-deep step
+// of a row is one 128-byte line:
+//   L^T (row-major M x Kp), V and R (column-major Kp x N); T is FP32 (row-major
+//   M x Np), and so is U unless stage B is explicit, which stores U split.
+// Offsets into a split array count padded elements: element (row, k) of a block
+// at `off` is at 2 (off + row Kp) + 16 (k / 8) + k % 8, its lo part 8 further.
 // Work decomposition as in the FP64 kernels: stage A one wave per 32 x 32
 // tile, stage C one workgroup per tile with the combine sum_j c_j T_j done on
 // the operand load and a 4-way split of the K iterations reduced through LDS.
@@ -41,18 +46,28 @@ __device__ inline void split8(const float (&x)[8], v8bf& hi, v8bf& lo) {
   }
 }
 
+__device__ inline void st8(__bf16* p, const v8bf& x) { *reinterpret_cast<v8bf*>(p) = x; }
+
 // Packed FP64 V columns -> padded split-BF16 copies (one workgroup per task of
-// at most 4096 padded elements).
+// at most 4096 padded elements, a group of 8 k per thread and round).
 __global__ __launch_bounds__(256) void k_split_v(const VConv* __restrict__ tasks, const double* __restrict__ vin,
-                                                 __bf16* __restrict__ Vhi, __bf16* __restrict__ Vlo) {
+                                                 __bf16* __restrict__ Vs) {
   const VConv t = tasks[blockIdx.x];
-  const int n = t.Kp * t.N;
+  const int g8 = t.Kp / 8, n = g8 * t.N;
   for (int e = threadIdx.x; e < n; e += 256) {
-    const int j = e / t.Kp, k = e - j * t.Kp;
-    const double x = (k < t.K) ? vin[t.src_off + (int64_t)j * t.K + k] : 0.0;
-    const __bf16 h = (__bf16)(float)x;
-    Vhi[t.dst_off + e] = h;
-    Vlo[t.dst_off + e] = (__bf16)(float)(x - (double)(float)h);
+    const int j = e / g8, k = 8 * (e - j * g8);
+    const double* __restrict__ src = vin + t.src_off + (int64_t)j * t.K + k;
+    v8bf hi, lo;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const double x = k + u < t.K ? src[u] : 0.0;
+      const __bf16 h = (__bf16)(float)x;
+      hi[u] = h;
+      lo[u] = (__bf16)(float)(x - (double)(float)h);
+    }
+    __bf16* __restrict__ dst = Vs + 2 * (t.dst_off + (int64_t)e * 8);
+    st8(dst, hi);
+    st8(dst + 8, lo);
   }
 }
 
@@ -60,15 +75,89 @@ __global__ __launch_bounds__(256) void k_split_v(const VConv* __restrict__ tasks
 // copies (L^T in the layout of k_split_v's output); one workgroup per task of
 // at most 4096 padded elements, task rows r read src[src_off + k M + r].
 __global__ __launch_bounds__(256) void k_split_lt(const VConv* __restrict__ tasks, const double* __restrict__ L,
-                                                  __bf16* __restrict__ Lhi, __bf16* __restrict__ Llo) {
+                                                  __bf16* __restrict__ Ls) {
   const VConv t = tasks[blockIdx.x];
-  const int n = t.Kp * t.N;
+  const int g8 = t.Kp / 8, n = g8 * t.N;
   for (int e = threadIdx.x; e < n; e += 256) {
-    const int r = e / t.Kp, k = e - r * t.Kp;
-    const double x = (k < t.K) ? L[t.src_off + (int64_t)k * t.pad + r] : 0.0;
-    const __bf16 h = (__bf16)(float)x;
-    Lhi[t.dst_off + e] = h;
-    Llo[t.dst_off + e] = (__bf16)(float)(x - (double)(float)h);
+    const int r = e / g8, k = 8 * (e - r * g8);
+    const double* __restrict__ src = L + t.src_off + (int64_t)k * t.pad + r;
+    v8bf hi, lo;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const double x = k + u < t.K ? src[(int64_t)u * t.pad] : 0.0;
+      const __bf16 h = (__bf16)(float)x;
+      hi[u] = h;
+      lo[u] = (__bf16)(float)(x - (double)(float)h);
+    }
+    __bf16* __restrict__ dst = Ls + 2 * (t.dst_off + (int64_t)e * 8);
+    st8(dst, hi);
+    st8(dst + 8, lo);
+  }
+}
+
+// Explicit stage B: U = sum_j c_j T_j, stored split (U's k is T's column), so
+// that stage C's tiles of one row of blocks load it instead of each splitting it
+// again.  One workgroup per task; a thread takes groups of 8 elements, the task's
+// terms come 64 at a time, one descriptor per lane, two terms per round.
+__global__ __launch_bounds__(256) void k_combine_split(const CombTask* __restrict__ tasks,
+                                                       const TermC16* __restrict__ terms,
+                                                       const float* __restrict__ Tbuf, __bf16* __restrict__ Us) {
+  constexpr int NV = kCombTaskElems / 256 / 8;
+  const CombTask t = tasks[blockIdx.x];
+  const int lane = threadIdx.x & 63;
+  const v4f zf = {0, 0, 0, 0};
+  v4f acc[NV][2];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) acc[v][0] = acc[v][1] = zf;
+  auto load = [&](const float* __restrict__ src, v4f (&x)[NV][2]) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int e = 8 * ((int)threadIdx.x + 256 * v);
+      x[v][0] = e < t.n ? *reinterpret_cast<const v4f*>(src + e) : zf;
+      x[v][1] = e < t.n ? *reinterpret_cast<const v4f*>(src + e + 4) : zf;
+    }
+  };
+  for (int g = t.term_begin; g < t.term_end; g += 64) {
+    const int nt = min(64, t.term_end - g);
+    int64_t my_off = 0;
+    float my_c = 0.f;
+    if (lane < nt) {
+      const TermC16 tm = terms[g + lane];
+      my_off = tm.t_off;
+      my_c = tm.c;
+    }
+    int j = 0;
+    for (; j + 1 < nt; j += 2) {
+      const float c0 = readlane_f(my_c, j), c1 = readlane_f(my_c, j + 1);
+      v4f x0[NV][2], x1[NV][2];
+      load(Tbuf + readlane64(my_off, j) + t.e0, x0);
+      load(Tbuf + readlane64(my_off, j + 1) + t.e0, x1);
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[v][q] += c0 * x0[v][q] + c1 * x1[v][q];
+    }
+    if (j < nt) {
+      const float c0 = readlane_f(my_c, j);
+      v4f x0[NV][2];
+      load(Tbuf + readlane64(my_off, j) + t.e0, x0);
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[v][q] += c0 * x0[v][q];
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int e = 8 * ((int)threadIdx.x + 256 * v);
+    if (e >= t.n) continue;
+    const float u[8] = {acc[v][0][0], acc[v][0][1], acc[v][0][2], acc[v][0][3],
+                        acc[v][1][0], acc[v][1][1], acc[v][1][2], acc[v][1][3]};
+    v8bf hi, lo;
+    split8(u, hi, lo);
+    __bf16* __restrict__ dst = Us + 2 * (t.u_off + t.e0 + e);
+    st8(dst, hi);
+    st8(dst + 8, lo);
   }
 }
 
@@ -117,8 +206,7 @@ __device__ inline TileCursor tile_at(const TileA16& d, int src) {
 }
 
 __global__ __launch_bounds__(256) void k_stage_a_bf16x3(const TileA16* __restrict__ tiles, int ntiles,
-                                                        const __bf16* __restrict__ Lhi, const __bf16* __restrict__ Llo,
-                                                        const __bf16* __restrict__ Vhi, const __bf16* __restrict__ Vlo,
+                                                        const __bf16* __restrict__ Ls, const __bf16* __restrict__ Vs,
                                                         float* __restrict__ Tp) {
   const int nwaves = gridDim.x * 4;
   const int w0 = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -132,14 +220,18 @@ __global__ __launch_bounds__(256) void k_stage_a_bf16x3(const TileA16* __restric
     const bool kin = k < t.Kp;
     const int i0 = t.m0 + li, i1 = i0 + 16, j0 = t.n0 + li, j1 = j0 + 16;
     const bool ra = kin && i0 < t.M, rb = kin && i1 < t.M, qa = kin && j0 < t.N, qb = kin && j1 < t.N;
-    o.a0h = ra ? ld8(Lhi + t.a_off + (int64_t)i0 * t.Kp + k) : z;
-    o.a0l = ra ? ld8(Llo + t.a_off + (int64_t)i0 * t.Kp + k) : z;
-    o.a1h = rb ? ld8(Lhi + t.a_off + (int64_t)i1 * t.Kp + k) : z;
-    o.a1l = rb ? ld8(Llo + t.a_off + (int64_t)i1 * t.Kp + k) : z;
-    o.b0h = qa ? ld8(Vhi + t.b_off + (int64_t)j0 * t.Kp + k) : z;
-    o.b0l = qa ? ld8(Vlo + t.b_off + (int64_t)j0 * t.Kp + k) : z;
-    o.b1h = qb ? ld8(Vhi + t.b_off + (int64_t)j1 * t.Kp + k) : z;
-    o.b1l = qb ? ld8(Vlo + t.b_off + (int64_t)j1 * t.Kp + k) : z;
+    const __bf16* __restrict__ pa0 = Ls + 2 * (t.a_off + (int64_t)i0 * t.Kp + k);
+    o.a0h = ra ? ld8(pa0) : z;
+    o.a0l = ra ? ld8(pa0 + 8) : z;
+    const __bf16* __restrict__ pa1 = Ls + 2 * (t.a_off + (int64_t)i1 * t.Kp + k);
+    o.a1h = rb ? ld8(pa1) : z;
+    o.a1l = rb ? ld8(pa1 + 8) : z;
+    const __bf16* __restrict__ pb0 = Vs + 2 * (t.b_off + (int64_t)j0 * t.Kp + k);
+    o.b0h = qa ? ld8(pb0) : z;
+    o.b0l = qa ? ld8(pb0 + 8) : z;
+    const __bf16* __restrict__ pb1 = Vs + 2 * (t.b_off + (int64_t)j1 * t.Kp + k);
+    o.b1h = qb ? ld8(pb1) : z;
+    o.b1l = qb ? ld8(pb1 + 8) : z;
   };
   auto store = [&](const TileCursor& t, const v4f& c00, const v4f& c01, const v4f& c10, const v4f& c11) {
     const int i0 = t.m0 + li, i1 = i0 + 16;
@@ -201,11 +293,13 @@ __global__ __launch_bounds__(256) void k_stage_a_bf16x3(const TileA16* __restric
   }
 }
 
-// Stage C: Vout (FP64 col-major M x N) = sum over chunks (sum_j c_j T_j) . R
+// Stage C, small problems: Vout (FP64 col-major M x N) = sum over chunks (sum_j c_j T_j) . R.
+// kSplitU (explicit stage B): every chunk reads one split block of unit weight from Us.
+template <bool kSplitU>
 __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict__ tiles, int ntiles,
                                                         const ChunkC16* __restrict__ chunks,
                                                         const TermC16* __restrict__ terms, const float* __restrict__ Tp,
-                                                        const __bf16* __restrict__ Rhi, const __bf16* __restrict__ Rlo,
+                                                        const __bf16* __restrict__ Us, const __bf16* __restrict__ Rs,
                                                         double* __restrict__ Vout) {
   __shared__ v4f red[3][4][64];
   if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
@@ -256,10 +350,24 @@ __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict_
         const int k = q * 32 + 8 * lg;
         const bool kin = k < Kp;
         const bool a0 = kin && r0, a1 = kin && r1;
-        const v8bf b0h = (kin && q0) ? ld8(Rhi + roff + (int64_t)j0 * Kp + k) : z;
-        const v8bf b0l = (kin && q0) ? ld8(Rlo + roff + (int64_t)j0 * Kp + k) : z;
-        const v8bf b1h = (kin && q1) ? ld8(Rhi + roff + (int64_t)j1 * Kp + k) : z;
-        const v8bf b1l = (kin && q1) ? ld8(Rlo + roff + (int64_t)j1 * Kp + k) : z;
+        const __bf16* __restrict__ p0 = Rs + 2 * (roff + (int64_t)j0 * Kp + k);
+        const __bf16* __restrict__ p1 = Rs + 2 * (roff + (int64_t)j1 * Kp + k);
+        WaveOps o;
+        o.b0h = (kin && q0) ? ld8(p0) : z;
+        o.b0l = (kin && q0) ? ld8(p0 + 8) : z;
+        o.b1h = (kin && q1) ? ld8(p1) : z;
+        o.b1l = (kin && q1) ? ld8(p1 + 8) : z;
+        if constexpr (kSplitU) {
+          const int64_t u = readlane64(my_toff, 0) + k;
+          const __bf16* __restrict__ u0 = Us + 2 * (u + (int64_t)i0 * Kp);
+          const __bf16* __restrict__ u1 = Us + 2 * (u + (int64_t)i1 * Kp);
+          o.a0h = a0 ? ld8(u0) : z;
+          o.a0l = a0 ? ld8(u0 + 8) : z;
+          o.a1h = a1 ? ld8(u1) : z;
+          o.a1l = a1 ? ld8(u1 + 8) : z;
+          wave_mac(o, has_m1, has_n1, c00, c01, c10, c11);
+          continue;
+        }
         float u0[8], u1[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -305,13 +413,8 @@ __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict_
             u1[e + 4] += c0 * x11[e];
           }
         }
-        WaveOps o;
         split8(u0, o.a0h, o.a0l);
         split8(u1, o.a1h, o.a1l);
-        o.b0h = b0h;
-        o.b0l = b0l;
-        o.b1h = b1h;
-        o.b1l = b1l;
         wave_mac(o, has_m1, has_n1, c00, c01, c10, c11);
       }
       it += nkb;
@@ -349,287 +452,341 @@ __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict_
 }
 
 // ---- LDS-staged 128 x 128 workgroup tiles for large blocks -------------------
-// 4 waves in a 2 x 2 grid, each owning 64 x 64 = 4 x 4 MFMA blocks.  Per
-// 64-deep K step the workgroup stages the split operand tiles A[128 x 64] and
-// B[64 x 128] (hi and lo) in LDS, k-contiguous with rows padded to 80
-// elements (16-byte aligned reads), and each wave then issues
-// 2 x 4 x 4 x 3 MFMAs from LDS reads.  The global loads of the next step are
-// in flight during those MFMAs.
+// 4 waves in a 2 x 2 grid, sub-blocks of 16 rows and columns dealt to the waves
+// alternately as in the FP64 kernels, and one of 16 instances NX x NY for the
+// tiles at a block's edge.  32-deep K steps, two LDS buffers: while a wave
+// multiplies step i from registers it reads step i + 1's operands from one buffer,
+// writes step i + 2's (loaded a step ago) to the other and issues the loads of
+// step i + 3, each between MFMAs; one barrier per step.
+//
+// What bounds it (12 products of 1152 x 1152 x 11520): MFMAs and barriers alone
+// run at 537 TFLOP/s of products (a third of the BF16 rate), with the LDS reads
+// 472, with the LDS writes 359; the loads then set the pace, by the number of
+// 64-byte requests to the L2, not by bytes: 246 with hi and lo in separate arrays
+// (64 bytes per row and step), 312 with the interleaved layout, whose rows are
+// whole 128-byte lines.  (A single-buffered 64-deep form with masked loads and
+// separate arrays: 278.)
 constexpr int kBT = kBigTile;
-constexpr int kBK = kBigK;
-// LDS row stride in bf16 elements: 160-byte rows (two workgroups of 80 KB
-// fill the CU's 160 KB); 3% faster than 144-byte rows on the C60 pivots
-constexpr int kLS = kBK + 16;
-constexpr int kPieces = kBT * kBK / 8 / 256;  // 16-byte pieces per operand tile and thread
+constexpr int kBKs = 32;            // k depth of a step
+constexpr int kLR = 2 * kBKs + 8;   // LDS row: 4 groups of [8 hi | 8 lo], 144 bytes: no bank conflicts
 
-struct BigSmem {
-  __bf16 Ah[kBT * kLS], Al[kBT * kLS], Bh[kBT * kLS], Bl[kBT * kLS];
+struct BigSmem {  // 72 KB, two workgroups per CU
+  __bf16 A[2][kBT * kLR], B[2][kBT * kLR];
 };
 
-// The wave raises its issue priority for its MFMA block (s_setprio), so that
-// a wave with operands in registers is served before the other workgroup's
-// waves staging their loads.
-__device__ inline void big_compute(const BigSmem& s, int wm, int wn, int li, int lg, v4f (&acc)[4][4]) {
-  __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-  for (int ks = 0; ks < kBK; ks += 32) {
-    v8bf ah[4], al[4], bh[4], bl[4];
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      ah[x] = *reinterpret_cast<const v8bf*>(&s.Ah[(wm + 16 * x + li) * kLS + ks + 8 * lg]);
-      al[x] = *reinterpret_cast<const v8bf*>(&s.Al[(wm + 16 * x + li) * kLS + ks + 8 * lg]);
-      bh[x] = *reinterpret_cast<const v8bf*>(&s.Bh[(wn + 16 * x + li) * kLS + ks + 8 * lg]);
-      bl[x] = *reinterpret_cast<const v8bf*>(&s.Bl[(wn + 16 * x + li) * kLS + ks + 8 * lg]);
-    }
-#pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-      for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = mac3(bh[ni], bl[ni], ah[mi], al[mi], acc[mi][ni]);
-  }
-  __builtin_amdgcn_s_setprio(0);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bf_buffer(const __bf16* p, bool on) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p), (short)0, on ? 0x7fffffff : 0, 0x00020000);
 }
 
-// thread tid's piece h of a staged operand tile: row (of A) / column (of B), k offset
-__device__ inline int piece_row(int tid, int h) { return (tid + 256 * h) / (kBK / 8); }
-__device__ inline int piece_k(int tid, int h) { return ((tid + 256 * h) % (kBK / 8)) * 8; }
+struct BigTile16 {
+  uint32_t offA[4], offB[4];  // byte offsets of this thread's pieces (rows row + 32 h) at k = 0
+  v8bf ra[4], rb[4];
+  const __bf16 *A, *B;        // wave-uniform: the tile's first row / column
+  int Kp, M, N, m0, n0;
+  int row, c8, kk;            // staging role: row, offset in the LDS row, first k of the piece
+  int kb;                     // k of the load cursor
+  int wm, wn, li, lg;
 
-__device__ inline void big_stage(BigSmem& s, int tid, const v8bf (&ah)[kPieces], const v8bf (&al)[kPieces],
-                                 const v8bf (&bh)[kPieces], const v8bf (&bl)[kPieces]) {
-#pragma unroll
-  for (int h = 0; h < kPieces; ++h) {
-    const int o = piece_row(tid, h) * kLS + piece_k(tid, h);
-    *reinterpret_cast<v8bf*>(&s.Ah[o]) = ah[h];
-    *reinterpret_cast<v8bf*>(&s.Al[o]) = al[h];
-    *reinterpret_cast<v8bf*>(&s.Bh[o]) = bh[h];
-    *reinterpret_cast<v8bf*>(&s.Bl[o]) = bl[h];
+  __device__ __forceinline__ void init(int M_, int N_, int mt, int nt, int tid) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    M = M_;
+    N = N_;
+    m0 = mt * kBT;
+    n0 = nt * kBT;
+    li = lane & 15;
+    lg = lane >> 4;
+    wm = (wave & 1) * 16;
+    wn = (wave >> 1) * 16;
+    row = tid >> 3;
+    c8 = (tid & 7) * 8;
+    kk = (tid & 6) * 4;
   }
+  __device__ __forceinline__ int nx() const { return min(4, (M - m0 + 31) / 32); }  // workgroup-uniform
+  __device__ __forceinline__ int ny() const { return min(4, (N - n0 + 31) / 32); }
+  // rows and columns past the block are clamped to its last one (not stored)
+  __device__ __forceinline__ void set(const __bf16* Ablk, const __bf16* Bblk, int Kp_) {
+    Kp = Kp_;
+    A = Ablk + 2 * (int64_t)m0 * Kp;
+    B = Bblk + 2 * (int64_t)n0 * Kp;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      offA[h] = 2u * (uint32_t)(min(row + 32 * h, M - 1 - m0) * 2 * Kp + c8);
+      offB[h] = 2u * (uint32_t)(min(row + 32 * h, N - 1 - n0) * 2 * Kp + c8);
+    }
+  }
+  // K step at kb: pieces at k >= Kp (a multiple of 8) load zeros
+  __device__ __forceinline__ void load_a(int kb) {
+    const auto r = bf_buffer(A + 2 * kb, kb < Kp);
+    const bool in = kb + kk < Kp;
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      ra[h] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(r, in ? offA[h] : 0x80000000u, 0, 0));
+  }
+  __device__ __forceinline__ void load_b(int kb) {
+    const auto r = bf_buffer(B + 2 * kb, kb < Kp);
+    const bool in = kb + kk < Kp;
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      rb[h] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(r, in ? offB[h] : 0x80000000u, 0, 0));
+  }
+  __device__ __forceinline__ void stage_a(BigSmem& s, int buf) const {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) st8(&s.A[buf][(row + 32 * h) * kLR + c8], ra[h]);
+  }
+  __device__ __forceinline__ void stage_b(BigSmem& s, int buf) const {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) st8(&s.B[buf][(row + 32 * h) * kLR + c8], rb[h]);
+  }
+};
+
+template <int NX, int NY>
+struct BigAcc16 {
+  v4f acc[NX][NY];
+  v8bf a[2][NX][2], b[2][NY][2];  // [step parity][sub-block][hi, lo]
+
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int y = 0; y < NY; ++y) acc[x][y] = v4f{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void read(const BigTile16& g, const BigSmem& s, int buf, int p) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+#pragma unroll
+      for (int x = 0; x < NX; ++x) a[p][x][q] = ld8(&s.A[buf][(g.wm + 32 * x + g.li) * kLR + 16 * g.lg + 8 * q]);
+#pragma unroll
+      for (int y = 0; y < NY; ++y) b[p][y][q] = ld8(&s.B[buf][(g.wn + 32 * y + g.li) * kLR + 16 * g.lg + 8 * q]);
+    }
+  }
+  __device__ __forceinline__ void mac(int p) {  // lo.hi, hi.lo, hi.hi, as mac3 adds them
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int y = 0; y < NY; ++y)
+          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[p][y][q == 0], a[p][x][q == 1], acc[x][y], 0, 0, 0);
+  }
+  // one step from registers p; buffer p ^ 1 holds the next one
+  template <class Next>
+  __device__ __forceinline__ void step(BigTile16& g, BigSmem& s, int p, Next&& next) {
+    next(g);          // the load cursor moves on
+    __syncthreads();  // the next step is staged, and this one's buffer no longer read
+    __builtin_amdgcn_sched_barrier(0);
+    read(g, s, p ^ 1, p ^ 1);
+    g.stage_a(s, p);
+    g.stage_b(s, p);
+    g.load_a(g.kb);
+    g.load_b(g.kb);
+    mac(p);
+#pragma unroll
+    for (int i = 0; i < 2 * (NX + NY); ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // global load
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // `steps` K steps; next(g) sets the operands and k of the following load (g.kb)
+  template <class Next>
+  __device__ __forceinline__ void run(BigTile16& g, BigSmem& s, int steps, Next&& next) {
+    zero();
+    if (steps <= 0) return;  // workgroup-uniform
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      if (i) {
+        g.stage_a(s, i - 1);
+        g.stage_b(s, i - 1);
+      }
+      next(g);
+      g.load_a(g.kb);
+      g.load_b(g.kb);
+    }
+    __syncthreads();
+    read(g, s, 0, 0);
+    for (int i = 0; i < steps; i += 2) {
+      step(g, s, 0, next);
+      if (i + 1 < steps) step(g, s, 1, next);
+    }
+  }
+};
+
+// f(BigAcc16 of the instance covering the tile); workgroup-uniform
+template <class F>
+__device__ __forceinline__ void with_big_acc16(const BigTile16& g, F&& f) {
+  const int nx = g.nx(), ny = g.ny();
+#define VMPS_BIG_ACC(X, Y)     \
+  if (nx == X && ny == Y) {    \
+    BigAcc16<X, Y> acc;        \
+    f(acc);                    \
+    return;                    \
+  }
+#define VMPS_BIG_ACC_ROW(X) VMPS_BIG_ACC(X, 1) VMPS_BIG_ACC(X, 2) VMPS_BIG_ACC(X, 3) VMPS_BIG_ACC(X, 4)
+  VMPS_BIG_ACC_ROW(1)
+  VMPS_BIG_ACC_ROW(2)
+  VMPS_BIG_ACC_ROW(3)
+  VMPS_BIG_ACC_ROW(4)
+#undef VMPS_BIG_ACC_ROW
+#undef VMPS_BIG_ACC
 }
 
 // Stage A, large problems: Tp (row-major M x Np) = Lt (row-major M x Kp) . V (col-major Kp x N)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_a_bf16x3_big(const TileA16* __restrict__ tiles, int ntiles,
-                                                            const __bf16* __restrict__ Lhi,
-                                                            const __bf16* __restrict__ Llo,
-                                                            const __bf16* __restrict__ Vhi,
-                                                            const __bf16* __restrict__ Vlo, float* __restrict__ Tp) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_a_bf16x3_big(
+    const TileA16* __restrict__ tiles, int ntiles, const __bf16* __restrict__ Ls, const __bf16* __restrict__ Vs,
+    float* __restrict__ Tp) {
   __shared__ BigSmem s;
   if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lg = lane >> 4;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
   const TileA16 t = tiles[blockIdx.x];
-  const int m0 = t.mt * kBT, n0 = t.nt * kBT;
-  const v8bf z = {};
-  v4f acc[4][4];
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = v4f{0, 0, 0, 0};
-  v8bf ah[kPieces], al[kPieces], bh[kPieces], bl[kPieces];
-  auto gload = [&](int kb) {
-#pragma unroll
-    for (int h = 0; h < kPieces; ++h) {
-      const int row = piece_row(tid, h), k = kb + piece_k(tid, h);
-      const bool ka = (m0 + row < t.M) && (k < t.Kp), kbv = (n0 + row < t.N) && (k < t.Kp);
-      ah[h] = ka ? ld8(Lhi + t.a_off + (int64_t)(m0 + row) * t.Kp + k) : z;
-      al[h] = ka ? ld8(Llo + t.a_off + (int64_t)(m0 + row) * t.Kp + k) : z;
-      bh[h] = kbv ? ld8(Vhi + t.b_off + (int64_t)(n0 + row) * t.Kp + k) : z;
-      bl[h] = kbv ? ld8(Vlo + t.b_off + (int64_t)(n0 + row) * t.Kp + k) : z;
-    }
-  };
-  gload(0);
-  for (int kb = 0; kb < t.Kp; kb += kBK) {
-    __syncthreads();  // the previous step's LDS reads are done
-    big_stage(s, tid, ah, al, bh, bl);
-    __syncthreads();
-    if (kb + kBK < t.Kp) gload(kb + kBK);  // in flight during the MFMAs below
-    big_compute(s, wm, wn, li, lg, acc);
-  }
+  if (t.Kp <= 0) return;  // a padding slot of the launch order (workgroup-uniform)
+  BigTile16 g;
+  g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
+  g.set(Ls + 2 * t.a_off, Vs + 2 * t.b_off, t.Kp);
   float* __restrict__ C = Tp + t.c_off;
+  with_big_acc16(g, [&](auto& acc) __attribute__((always_inline)) {
+    g.kb = -kBKs;
+    acc.run(g, s, (t.Kp + kBKs - 1) / kBKs, [](BigTile16& h) __attribute__((always_inline)) { h.kb += kBKs; });
+    constexpr int NX = sizeof(acc.acc) / sizeof(acc.acc[0]), NY = sizeof(acc.acc[0]) / sizeof(v4f);
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
-    const int i = m0 + wm + 16 * mi + li;
-    if (i >= t.M) continue;
+    for (int x = 0; x < NX; ++x) {
+      const int i = g.m0 + g.wm + 32 * x + g.li;
+      if (i >= t.M) continue;
 #pragma unroll
-    for (int ni = 0; ni < 4; ++ni)
+      for (int y = 0; y < NY; ++y) {
+        const int j = g.n0 + g.wn + 32 * y + 4 * g.lg;  // Np and c_off are multiples of 8: 16-byte aligned
+        float* __restrict__ c = C + (int64_t)i * t.Np + j;
+        if (j + 4 <= t.N) {
+          *reinterpret_cast<v4f*>(c) = acc.acc[x][y];
+        } else {  // the padding columns keep their zeros
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int j = n0 + wn + 16 * ni + 4 * lg + v;
-        if (j < t.N) C[(int64_t)i * t.Np + j] = acc[mi][ni][v];
+          for (int v = 0; v < 4; ++v)
+            if (j + v < t.N) c[v] = acc.acc[x][y][v];
+        }
       }
-  }
+    }
+  });
 }
 
 // Stage C, large output blocks: Vout (FP64 col-major M x N) = sum_chunks (sum_j c_j T_j) . R.
-// Work item w covers iterations [it_begin, it_end) of its tile's flattened
-// (chunk, kBK-deep k block) loop; with slot >= 0 it writes an FP32 partial tile
-// (column-major 128 x 128) that k_reduce_partials sums in slot order.
-// kOneTerm: every chunk has one term (explicit stage B): streamed with the
-// next K step's loads in flight (a separate instantiation, see k_stage_c_big)
-template <bool kOneTerm>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_bf16x3_big(const TileC* __restrict__ tiles,
-                                                            const int32_t* __restrict__ w_tile,
-                                                            const int32_t* __restrict__ w_begin,
-                                                            const int32_t* __restrict__ w_end,
-                                                            const int64_t* __restrict__ w_slot, int nwork,
-                                                            const ChunkC16* __restrict__ chunks,
-                                                            const TermC16* __restrict__ terms,
-                                                            const float* __restrict__ Tp,
-                                                            const __bf16* __restrict__ Rhi,
-                                                            const __bf16* __restrict__ Rlo,
-                                                            double* __restrict__ Vout, float* __restrict__ partial) {
+// Work items as in the FP64 kernel (BigItemC, in steps of kBKs k); partial
+// tiles are FP32, column-major 128 x 128.
+// kSplitU (explicit stage B): every chunk reads one split block of unit weight
+// from Us, the loads running ahead across the chunks' boundaries; otherwise U
+// is formed and split on the operand load.
+template <bool kSplitU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_bf16x3_big(
+    const TileC* __restrict__ tiles, const BigItemC* __restrict__ items, int nitems,
+    const ChunkC16* __restrict__ chunks, const TermC16* __restrict__ terms, const float* __restrict__ Tp,
+    const __bf16* __restrict__ Us, const __bf16* __restrict__ Rs, double* __restrict__ Vout,
+    float* __restrict__ partial) {
   __shared__ BigSmem s;
-  if ((int)blockIdx.x >= nwork) return;  // workgroup-uniform
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lg = lane >> 4;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-  const TileC t = tiles[w_tile[blockIdx.x]];
-  const int it0 = w_begin[blockIdx.x], it1 = w_end[blockIdx.x];
-  const int64_t slot = w_slot[blockIdx.x];
-  const int m0 = t.mt * kBT, n0 = t.nt * kBT;
-  const v8bf z = {};
-  const v4f zf = {0, 0, 0, 0};
-  v4f acc[4][4];
+  if ((int)blockIdx.x >= nitems) return;  // workgroup-uniform
+  const BigItemC w = items[blockIdx.x];
+  if (w.tile < 0) return;  // a padding slot of the launch order (workgroup-uniform)
+  const TileC t = tiles[w.tile];
+  BigTile16 g;
+  g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
+  int left = w.nsteps, c = w.chunk, kb = w.step * kBKs;
+  auto store = [&](auto& acc) __attribute__((always_inline)) {
+    constexpr int NX = sizeof(acc.acc) / sizeof(acc.acc[0]), NY = sizeof(acc.acc[0]) / sizeof(v4f);
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+    for (int x = 0; x < NX; ++x) {
+      const int r = g.wm + 32 * x + g.li;
+      if (g.m0 + r >= t.M) continue;
 #pragma unroll
-    for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = zf;
-  int it = 0;
-  for (int c = t.chunk_begin; c < t.chunk_end && it < it1; ++c) {
-    const ChunkC16 ch = chunks[c];
-    const int nsteps = (ch.Kp + kBK - 1) / kBK;
-    if (it + nsteps <= it0) {
-      it += nsteps;
-      continue;
-    }
-    // the chunk's terms (at most 64), one per lane, broadcast with readlane
-    const int nt = ch.term_end - ch.term_begin;
-    int64_t my_toff = 0;
-    float my_c = 0.f;
-    if (lane < nt) {
-      const TermC16 tm = terms[ch.term_begin + lane];
-      my_toff = tm.t_off;
-      my_c = tm.c;
-    }
-    if (kOneTerm) {  // one term (explicit stage B): a plain product, next step's loads in flight
-      const float* __restrict__ T0 = Tp + readlane64(my_toff, 0);
-      const float c0 = readlane_f(my_c, 0);
-      const int s_lo = max(0, it0 - it), s_hi = min(nsteps, it1 - it);  // this work item's K steps
-      v4f xr[kPieces][2];
-      v8bf bh[kPieces], bl[kPieces];
-      auto gload = [&](int kb) {
+      for (int y = 0; y < NY; ++y)
 #pragma unroll
-        for (int h = 0; h < kPieces; ++h) {
-          const int row = piece_row(tid, h), k = kb + piece_k(tid, h);
-          const bool ka = (m0 + row < t.M) && (k < ch.Kp), kbv = (n0 + row < t.N) && (k < ch.Kp);
-          const float* __restrict__ src = T0 + (int64_t)(m0 + row) * ch.Kp + k;
-          xr[h][0] = ka ? *reinterpret_cast<const v4f*>(src) : zf;
-          xr[h][1] = ka ? *reinterpret_cast<const v4f*>(src + 4) : zf;
-          bh[h] = kbv ? ld8(Rhi + ch.r_off + (int64_t)(n0 + row) * ch.Kp + k) : z;
-          bl[h] = kbv ? ld8(Rlo + ch.r_off + (int64_t)(n0 + row) * ch.Kp + k) : z;
+        for (int v = 0; v < 4; ++v) {
+          const int cl = g.wn + 32 * y + 4 * g.lg + v;
+          if (g.n0 + cl >= t.N) continue;
+          if (w.slot < 0)
+            Vout[t.c_off + (int64_t)(g.n0 + cl) * t.M + g.m0 + r] = (double)acc.acc[x][y][v];
+          else
+            partial[w.slot * (int64_t)(kBT * kBT) + cl * kBT + r] = acc.acc[x][y][v];
         }
-      };
-      if (s_lo < s_hi) gload(s_lo * kBK);
-      for (int st = s_lo; st < s_hi; ++st) {
-        v8bf ah[kPieces], al[kPieces];
+    }
+  };
+  if constexpr (kSplitU) {
+    g.kb = kb - kBKs;
+    auto enter = [&](BigTile16& h) __attribute__((always_inline)) {
+      const ChunkC16 ch = chunks[c];
+      h.set(Us + 2 * terms[ch.term_begin].t_off, Rs + 2 * ch.r_off, ch.Kp);
+    };
+    if (left > 0) enter(g);
+    with_big_acc16(g, [&](auto& acc) __attribute__((always_inline)) {
+      acc.run(g, s, w.nsteps, [&](BigTile16& h) __attribute__((always_inline)) {
+        h.kb += kBKs;
+        while (h.kb >= h.Kp && left > 0) {
+          ++c;
+          h.kb = 0;
+          enter(h);
+        }
+        --left;
+      });
+      store(acc);
+    });
+  } else {
+    const int lane = threadIdx.x & 63;
+    BigAcc16<4, 4> acc;
+    acc.zero();
+    const int row = threadIdx.x >> 2, k8 = (threadIdx.x & 3) * 8;  // U pieces: rows row, row + 64, 8 k each
+    for (; left > 0; ++c, kb = 0) {
+      const ChunkC16 ch = chunks[c];
+      const int nt = ch.term_end - ch.term_begin;
+      int64_t my_toff = 0;
+      float my_c = 0.f;
+      if (lane < nt) {
+        const TermC16 tm = terms[ch.term_begin + lane];
+        my_toff = tm.t_off;
+        my_c = tm.c;
+      }
+      g.set(Rs, Rs + 2 * ch.r_off, ch.Kp);  // A is not used
+      for (; kb < ch.Kp && left > 0; kb += kBKs, --left) {
+        const v4f zf = {0, 0, 0, 0};
+        v4f u[2][2] = {{zf, zf}, {zf, zf}};
+        bool in[2];
+        int64_t at[2];
 #pragma unroll
-        for (int h = 0; h < kPieces; ++h) {
-          float u[8];
+        for (int h = 0; h < 2; ++h) {
+          in[h] = g.m0 + row + 64 * h < t.M && kb + k8 < ch.Kp;
+          at[h] = (int64_t)(g.m0 + row + 64 * h) * ch.Kp + kb + k8;
+        }
+        g.load_b(kb);
+        for (int jt = 0; jt < nt; ++jt) {
+          const float* __restrict__ T0 = Tp + readlane64(my_toff, jt);
+          const float c0 = readlane_f(my_c, jt);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            u[e] = c0 * xr[h][0][e];
-            u[e + 4] = c0 * xr[h][1][e];
+          for (int h = 0; h < 2; ++h) {
+            u[h][0] += c0 * (in[h] ? *reinterpret_cast<const v4f*>(T0 + at[h]) : zf);
+            u[h][1] += c0 * (in[h] ? *reinterpret_cast<const v4f*>(T0 + at[h] + 4) : zf);
           }
-          split8(u, ah[h], al[h]);
         }
         __syncthreads();  // the previous step's LDS reads are done
-        big_stage(s, tid, ah, al, bh, bl);
-        __syncthreads();
-        if (st + 1 < s_hi) gload((st + 1) * kBK);
-        big_compute(s, wm, wn, li, lg, acc);
-      }
-      it += nsteps;
-      continue;
-    }
-    for (int kb = 0; kb < ch.Kp; kb += kBK, ++it) {
-      if (it < it0 || it >= it1) continue;  // workgroup-uniform
-      v8bf ah[kPieces], al[kPieces], bh[kPieces], bl[kPieces];
-      bool ka[kPieces];
-      int64_t arow[kPieces];
-      float u[kPieces][8];
+        g.stage_b(s, 0);
 #pragma unroll
-      for (int h = 0; h < kPieces; ++h) {
-        const int row = piece_row(tid, h), k = kb + piece_k(tid, h);
-        ka[h] = (m0 + row < t.M) && (k < ch.Kp);
-        arow[h] = (int64_t)(m0 + row) * ch.Kp + k;
-        const bool kbv = (n0 + row < t.N) && (k < ch.Kp);
-        bh[h] = kbv ? ld8(Rhi + ch.r_off + (int64_t)(n0 + row) * ch.Kp + k) : z;
-        bl[h] = kbv ? ld8(Rlo + ch.r_off + (int64_t)(n0 + row) * ch.Kp + k) : z;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) u[h][e] = 0.f;
-      }
-      // U = sum_j c_j T_j on this thread's 8-wide row pieces
-      for (int jt = 0; jt < nt; ++jt) {
-        const float* __restrict__ T0 = Tp + readlane64(my_toff, jt);
-        const float c0 = readlane_f(my_c, jt);
-        v4f x[kPieces][2];
-#pragma unroll
-        for (int h = 0; h < kPieces; ++h) {
-          x[h][0] = ka[h] ? *reinterpret_cast<const v4f*>(T0 + arow[h]) : zf;
-          x[h][1] = ka[h] ? *reinterpret_cast<const v4f*>(T0 + arow[h] + 4) : zf;
+        for (int h = 0; h < 2; ++h) {
+          const float x[8] = {u[h][0][0], u[h][0][1], u[h][0][2], u[h][0][3],
+                              u[h][1][0], u[h][1][1], u[h][1][2], u[h][1][3]};
+          v8bf hi, lo;
+          split8(x, hi, lo);
+          st8(&s.A[0][(row + 64 * h) * kLR + 2 * k8], hi);
+          st8(&s.A[0][(row + 64 * h) * kLR + 2 * k8 + 8], lo);
         }
-#pragma unroll
-        for (int h = 0; h < kPieces; ++h)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            u[h][e] += c0 * x[h][0][e];
-            u[h][e + 4] += c0 * x[h][1][e];
-          }
+        __syncthreads();
+        acc.read(g, s, 0, 0);
+        acc.mac(0);
       }
-#pragma unroll
-      for (int h = 0; h < kPieces; ++h) split8(u[h], ah[h], al[h]);
-      __syncthreads();
-      big_stage(s, tid, ah, al, bh, bl);
-      __syncthreads();
-      big_compute(s, wm, wn, li, lg, acc);
     }
-  }
-  double* __restrict__ C = Vout + t.c_off;
-  float* __restrict__ P = partial + (slot < 0 ? 0 : slot * (int64_t)(kBT * kBT));
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
-    const int r = wm + 16 * mi + li, i = m0 + r;
-    if (i >= t.M) continue;
-#pragma unroll
-    for (int ni = 0; ni < 4; ++ni)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int cl = wn + 16 * ni + 4 * lg + v, j = n0 + cl;
-        if (j >= t.N) continue;
-        if (slot < 0)
-          C[(int64_t)j * t.M + i] = (double)acc[mi][ni][v];
-        else
-          P[cl * kBT + r] = acc[mi][ni][v];
-      }
-  }
-}
-
-// Vout tile = sum over its split partials, in slot order.
-__global__ __launch_bounds__(256) void k_reduce_partials(const TileC* __restrict__ tiles,
-                                                         const int32_t* __restrict__ r_tile,
-                                                         const int64_t* __restrict__ r_slot,
-                                                         const int32_t* __restrict__ r_nsplit,
-                                                         const float* __restrict__ partial, double* __restrict__ Vout) {
-  const TileC t = tiles[r_tile[blockIdx.x]];
-  const int64_t s0 = r_slot[blockIdx.x];
-  const int ns = r_nsplit[blockIdx.x];
-  const int m0 = t.mt * kBT, n0 = t.nt * kBT;
-  for (int e = threadIdx.x; e < kBT * kBT; e += 256) {
-    const int cl = e / kBT, r = e - cl * kBT;
-    const int i = m0 + r, j = n0 + cl;
-    if (i >= t.M || j >= t.N) continue;
-    float acc = 0.f;
-    for (int s = 0; s < ns; ++s) acc += partial[(s0 + s) * (int64_t)(kBT * kBT) + e];
-    Vout[t.c_off + (int64_t)j * t.M + i] = (double)acc;
+    store(acc);
   }
 }
 
@@ -639,25 +796,20 @@ void DevPlan::ensure_bf16_buffers() {
   if (bf16_ready || (H.tilesA.empty() && H.tilesC.empty())) return;
   Bf16Layout B;
   build_bf16_layout(H, B);  // work lists; the operands are split on the device
-  Lhi.alloc(std::max<int64_t>(1, B.L_size));
-  Llo.alloc(std::max<int64_t>(1, B.L_size));
-  Rhi.alloc(std::max<int64_t>(1, B.R_size));
-  Rlo.alloc(std::max<int64_t>(1, B.R_size));
+  Ls.alloc(std::max<int64_t>(1, 2 * B.L_size));
+  Rs.alloc(std::max<int64_t>(1, 2 * B.R_size));
   {
     DevBuf<VConv> lc, rc;  // freed after the synchronisation below
     lc.upload(B.lconv, stream);
     rc.upload(B.rconv, stream);
     if (lc.n)
-      hipLaunchKernelGGL(k_split_lt, dim3((unsigned)lc.n), dim3(256), 0, stream, lc.p, L.p, (__bf16*)Lhi.p,
-                         (__bf16*)Llo.p);
+      hipLaunchKernelGGL(k_split_lt, dim3((unsigned)lc.n), dim3(256), 0, stream, lc.p, L.p, (__bf16*)Ls.p);
     if (rc.n)
-      hipLaunchKernelGGL(k_split_v, dim3((unsigned)rc.n), dim3(256), 0, stream, rc.p, R.p, (__bf16*)Rhi.p,
-                         (__bf16*)Rlo.p);
+      hipLaunchKernelGGL(k_split_v, dim3((unsigned)rc.n), dim3(256), 0, stream, rc.p, R.p, (__bf16*)Rs.p);
     VMPS_HIP_CHECK(hipGetLastError());
     VMPS_HIP_CHECK(hipStreamSynchronize(stream));
   }
-  Vhi.alloc(std::max<int64_t>(1, B.V_size));
-  Vlo.alloc(std::max<int64_t>(1, B.V_size));
+  Vs.alloc(std::max<int64_t>(1, 2 * B.V_size));
   Tp.alloc(std::max<int64_t>(1, B.T_size));
   VMPS_HIP_CHECK(hipMemsetAsync(Tp.p, 0, Tp.n * sizeof(float), stream));  // padding columns stay zero
   upload_bf16_lists(B);
@@ -672,23 +824,18 @@ void DevPlan::upload_bf16_lists(const Bf16Layout& B) {
   bfAbig.upload(B.tilesA_big, stream);
   bfCsmall.upload(B.tilesC_small, stream);
   bfCbig.upload(B.tilesC_big, stream);
-  wTile.upload(B.splitC_tile, stream);
-  wBegin.upload(B.splitC_begin, stream);
-  wEnd.upload(B.splitC_end, stream);
-  wSlot.upload(B.splitC_slot, stream);
-  rTile.upload(B.redC_tile, stream);
-  rSlot.upload(B.redC_slot, stream);
-  rNs.upload(B.redC_nsplit, stream);
-  Cpart.alloc(std::max<int64_t>(1, B.partial_slots) * (int64_t)kBigTile * kBigTile);
+  itemsC16.upload(B.itemsC, stream);
+  redsC16.upload(B.redsC, stream);
+  if (Cpart.n < (size_t)(B.slotsC * kBigTile * kBigTile)) Cpart.alloc((size_t)(B.slotsC * kBigTile * kBigTile));
   bfC.upload(B.chunksC, stream);
   bfT.upload(B.termsC, stream);
   vconv.upload(B.vconv, stream);
   bfCombTasks.upload(B.comb_tasks, stream);
   bfCombTerms.upload(B.comb_terms, stream);
   if (H.explicit_u)
-    Up.alloc(std::max<int64_t>(1, B.U_size));
+    Us.alloc(std::max<int64_t>(1, 2 * B.U_size));
   else
-    Up.release();
+    Us.release();
 }
 
 void DevPlan::retile(int wave_edge, int big_min, int big_min64, bool explicit_u) {
@@ -713,40 +860,35 @@ void DevPlan::retile(int wave_edge, int big_min, int big_min64, bool explicit_u)
 }
 
 void DevPlan::launch_stage_bf16x3(int stage, const double* d_vin, double* d_vout, hipStream_t s) {
-  const int nA = (int)bfA.n, nAb = (int)bfAbig.n, nC = (int)bfCsmall.n, nCb = (int)bfCbig.n;
+  const int nA = (int)bfA.n, nAb = (int)bfAbig.n, nC = (int)bfCsmall.n, nW = (int)itemsC16.n, nR = (int)redsC16.n;
+  const __bf16 *l = (const __bf16*)Ls.p, *r = (const __bf16*)Rs.p, *v = (const __bf16*)Vs.p, *u = (const __bf16*)Us.p;
   if (stage == 0) {
     if (vconv.n)
-      hipLaunchKernelGGL(k_split_v, dim3((unsigned)vconv.n), dim3(256), 0, s, vconv.p, d_vin, (__bf16*)Vhi.p,
-                         (__bf16*)Vlo.p);
+      hipLaunchKernelGGL(k_split_v, dim3((unsigned)vconv.n), dim3(256), 0, s, vconv.p, d_vin, (__bf16*)Vs.p);
     if (nAb)
-      hipLaunchKernelGGL(k_stage_a_bf16x3_big, dim3((unsigned)nAb), dim3(256), 0, s, bfAbig.p, nAb,
-                         (const __bf16*)Lhi.p, (const __bf16*)Llo.p, (const __bf16*)Vhi.p, (const __bf16*)Vlo.p, Tp.p);
+      hipLaunchKernelGGL(k_stage_a_bf16x3_big, dim3((unsigned)nAb), dim3(256), 0, s, bfAbig.p, nAb, l, v, Tp.p);
     if (nA)
       hipLaunchKernelGGL(k_stage_a_bf16x3, dim3((unsigned)persistent_blocks(nA, occ_a16)), dim3(256), 0, s, bfA.p, nA,
-                         (const __bf16*)Lhi.p, (const __bf16*)Llo.p, (const __bf16*)Vhi.p, (const __bf16*)Vlo.p, Tp.p);
+                         l, v, Tp.p);
   } else if (stage == 2) {
-    const int nW = (int)wTile.n, nR = (int)rTile.n;
-    const float* src = Tp.p;
-    if (H.explicit_u) {  // stage B: U = sum c T, then stage C reads U
-      if (bfCombTasks.n)
-        hipLaunchKernelGGL((k_combine<float, TermC16>), dim3((unsigned)bfCombTasks.n), dim3(256), 0, s,
-                           bfCombTasks.p, bfCombTerms.p, Tp.p, Up.p);
-      src = Up.p;
-    }
-    if (nCb && nW && H.explicit_u)
-      hipLaunchKernelGGL(k_stage_c_bf16x3_big<true>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, wTile.p,
-                         wBegin.p, wEnd.p, wSlot.p, nW, bfC.p, bfT.p, src, (const __bf16*)Rhi.p, (const __bf16*)Rlo.p,
-                         d_vout, Cpart.p);
-    else if (nCb && nW)
-      hipLaunchKernelGGL(k_stage_c_bf16x3_big<false>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, wTile.p,
-                         wBegin.p, wEnd.p, wSlot.p, nW, bfC.p, bfT.p, src, (const __bf16*)Rhi.p, (const __bf16*)Rlo.p,
-                         d_vout, Cpart.p);
+    if (H.explicit_u && bfCombTasks.n)  // stage B: U = sum c T, then stage C reads U
+      hipLaunchKernelGGL(k_combine_split, dim3((unsigned)bfCombTasks.n), dim3(256), 0, s, bfCombTasks.p,
+                         bfCombTerms.p, Tp.p, (__bf16*)Us.p);
+    if (nW && H.explicit_u)
+      hipLaunchKernelGGL(k_stage_c_bf16x3_big<true>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p, nW,
+                         bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
+    else if (nW)
+      hipLaunchKernelGGL(k_stage_c_bf16x3_big<false>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p, nW,
+                         bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
     if (nR)
-      hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)nR), dim3(256), 0, s, bfCbig.p, rTile.p, rSlot.p, rNs.p,
-                         Cpart.p, d_vout);
-    if (nC)
-      hipLaunchKernelGGL(k_stage_c_bf16x3, dim3((unsigned)nC), dim3(256), 0, s, bfCsmall.p, nC, bfC.p, bfT.p, src,
-                         (const __bf16*)Rhi.p, (const __bf16*)Rlo.p, d_vout);
+      hipLaunchKernelGGL((k_reduce_big<float, double, kBigTile>), dim3((unsigned)(4 * nR)), dim3(256), 0, s, bfCbig.p,
+                         redsC16.p, Cpart.p, d_vout);
+    if (nC && H.explicit_u)
+      hipLaunchKernelGGL(k_stage_c_bf16x3<true>, dim3((unsigned)nC), dim3(256), 0, s, bfCsmall.p, nC, bfC.p, bfT.p,
+                         Tp.p, u, r, d_vout);
+    else if (nC)
+      hipLaunchKernelGGL(k_stage_c_bf16x3<false>, dim3((unsigned)nC), dim3(256), 0, s, bfCsmall.p, nC, bfC.p, bfT.p,
+                         Tp.p, u, r, d_vout);
   }
   VMPS_HIP_CHECK(hipGetLastError());
 }

@@ -727,17 +727,20 @@ void interleave_queues(const std::vector<std::vector<T>>& queue, const T& paddin
 // ignored the supertiles took 22 ms instead of 12).  Parts get smaller towards
 // the end of a queue: half, then a quarter, then a twelfth of the work that one
 // of the workgroups resident at once has in all.
-void build_big_items(HostPlan& H) {
-  constexpr int64_t kStep = 16, kCu = 256, kMinSteps = 16;
-  const int e = H.big_edge, u = e / 32;
-  H.itemsC_b.clear();
-  H.redsC_b.clear();
-  H.slotsC_b = 0;
-  const size_t n = H.tilesC_b.size();
+// `kstep`: k depth of a step; `resident`: workgroups per CU; parts keep at least
+// `min_steps` steps, of about 8 microseconds together.
+void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks, int e, int64_t kstep,
+                     int resident, int64_t min_steps, std::vector<BigItemC>& out, std::vector<BigRedC>& reds,
+                     int64_t& slots) {
+  constexpr int64_t kCu = 256;
+  const int u = e / 32;
+  reds.clear();
+  slots = 0;
+  const size_t n = tiles.size();
   std::vector<int64_t> steps(n, 0), unit(n, 0);
   for (size_t i = 0; i < n; ++i) {
-    const TileC& t = H.tilesC_b[i];
-    for (int32_t c = t.chunk_begin; c < t.chunk_end; ++c) steps[i] += (H.chunksC[c].K + kStep - 1) / kStep;
+    const TileC& t = tiles[i];
+    for (int32_t c = t.chunk_begin; c < t.chunk_end; ++c) steps[i] += (chunks[c].K + kstep - 1) / kstep;
     // a step's MFMAs in 32 x 32 units, plus its barrier and staging
     unit[i] = std::min<int64_t>(u, (t.M - t.mt * e + 31) / 32) * std::min<int64_t>(u, (t.N - t.nt * e + 31) / 32) + 1;
   }
@@ -747,7 +750,7 @@ void build_big_items(HostPlan& H) {
     super.clear();
     std::map<std::array<int64_t, 3>, size_t> id;
     for (size_t i = 0; i < n; ++i) {
-      const TileC& t = H.tilesC_b[i];
+      const TileC& t = tiles[i];
       auto it = id.emplace(std::array<int64_t, 3>{t.c_off, t.mt / edge, t.nt / edge}, super.size());
       if (it.second) super.emplace_back();
       super[it.first->second].push_back((int64_t)i);
@@ -759,7 +762,7 @@ void build_big_items(HostPlan& H) {
     group[g] = (int64_t)g;
     for (int64_t i : super[g]) cost[g] += steps[i] * unit[i];
   }
-  const double resident = (double)(kCu / kXcdCount) * (e == 64 ? 3 : 2);
+  const double per_xcd = (double)(kCu / kXcdCount) * resident;
   std::vector<std::vector<BigItemC>> items(kXcdCount);
   const std::vector<std::vector<int64_t>> queue = xcd_queues(group, cost);
   for (int x = 0; x < kXcdCount; ++x) {
@@ -767,38 +770,38 @@ void build_big_items(HostPlan& H) {
     for (int64_t g : queue[x]) total += (double)cost[g];
     for (int64_t g : queue[x]) {
       const double f = total > 0 ? done / total : 0.0;
-      const double most = std::max(1.0, total / resident * (f < 0.5 ? 0.5 : f < 0.8 ? 0.25 : 1.0 / 12));
+      const double most = std::max(1.0, total / per_xcd * (f < 0.5 ? 0.5 : f < 0.8 ? 0.25 : 1.0 / 12));
       int64_t S = 1, fewest = std::numeric_limits<int64_t>::max();
       for (int64_t i : super[g]) {
         S = std::max(S, (int64_t)std::ceil((double)(steps[i] * unit[i]) / most));
         fewest = std::min(fewest, steps[i]);
       }
-      S = std::max<int64_t>(1, std::min(S, fewest / kMinSteps));
+      S = std::max<int64_t>(1, std::min(S, fewest / min_steps));
       std::vector<std::array<int64_t, 2>> at;  // (chunk, step within it) where the next part of a tile starts
-      for (int64_t i : super[g]) at.push_back({H.tilesC_b[i].chunk_begin, 0});
+      for (int64_t i : super[g]) at.push_back({tiles[i].chunk_begin, 0});
       for (int64_t p = 0; p < S; ++p)
         for (size_t j = 0; j < super[g].size(); ++j) {
           const int64_t i = super[g][j];
-          const TileC& t = H.tilesC_b[i];
+          const TileC& t = tiles[i];
           const int64_t k = steps[i] * (p + 1) / S - steps[i] * p / S;
           int64_t &c = at[j][0], &st = at[j][1];
           items[x].push_back({(int32_t)i, (int32_t)c, (int32_t)st, (int32_t)k,
-                              S > 1 ? H.slotsC_b + (int64_t)j * S + p : -1});
+                              S > 1 ? slots + (int64_t)j * S + p : -1});
           for (st += k; c < t.chunk_end; ++c) {
-            const int64_t nc = (H.chunksC[c].K + kStep - 1) / kStep;
+            const int64_t nc = (chunks[c].K + kstep - 1) / kstep;
             if (st < nc) break;
             st -= nc;
           }
         }
       if (S > 1)
         for (size_t j = 0; j < super[g].size(); ++j) {
-          H.redsC_b.push_back({H.slotsC_b, (int32_t)super[g][j], (int32_t)S});
-          H.slotsC_b += S;
+          reds.push_back({slots, (int32_t)super[g][j], (int32_t)S});
+          slots += S;
         }
       done += (double)cost[g];
     }
   }
-  interleave_queues(items, BigItemC{-1, 0, 0, 0, -1}, H.itemsC_b);
+  interleave_queues(items, BigItemC{-1, 0, 0, 0, -1}, out);
 }
 
 int choose_wave_edge(const HostPlan& H) {
@@ -829,7 +832,8 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
     H.big_edge = tiles128 >= 256 ? 128 : 64;
     make_tiles(H, H.big_edge, H.crange, H.tilesA_b, H.tilesC_b, big_min64);
     order_for_xcds(H.tilesA_b);
-    build_big_items(H);
+    build_big_items(H.tilesC_b, H.chunksC, H.big_edge, 16, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b, H.redsC_b,
+                    H.slotsC_b);
   } else {
     H.tilesA_b.clear();
     H.tilesC_b.clear();
@@ -1195,16 +1199,17 @@ void build_plan_tables(const TripleSet& S, HostPlan& H) {
   }
 
   validate_host_plan(H);
-  // Pivots with blocks of 256 and more start from the explicit stage B and
-  // the FP64 / FP32 LDS-staged tiles for every problem, which the autotuner
-  // picks on every such pivot measured; the tuner then finds the lists already
-  // built for its first candidate instead of building them a second time.
+  // Pivots with blocks of 256 and more take the explicit stage B and the
+  // LDS-staged tiles for every problem, in every precision.
   // For every problem, since a second launch for the small blocks runs on a
   // nearly empty chip: with blocks below 128 or 32 on wave tiles the U(1) chain at
   // M = 2048 took 283 or 281 instead of 263 us, C60 at M = 1024 780 or 709
-  // instead of 676 us.
+  // instead of 676 us; split-BF16 with blocks below 96 or all on wave tiles 110
+  // or 151 instead of 96 us and 274 or 358 instead of 242 us (C60 at M = 4096:
+  // 5.6 instead of 5.5 ms for 96).
   if (st.max_block_dim >= 2 * kBigTile) {
     H.explicit_u = true;
+    H.big_min = 1;
     if (H.big_min64 <= 0) H.big_min64 = 1;
   }
   build_tiles(H);
@@ -1332,80 +1337,20 @@ void build_bf16_layout(const HostPlan& H, Bf16Layout& B) {
       B.tilesC_big.push_back(b);
     }
   }
-  // Split the K iterations of a big stage C tile over several workgroups only
-  // when the big tiles alone cannot fill the GPU (the FP32 partials cost a
-  // round trip through HBM): aim at ~512 workgroups, at least 8 iterations of
-  // kBigK k per split, at most 4 splits.
-  const int64_t nbig = (int64_t)B.tilesC_big.size();
-  const int64_t want = nbig > 0 ? std::max<int64_t>(1, std::min<int64_t>(4, 512 / nbig)) : 1;
-  for (size_t ti = 0; ti < B.tilesC_big.size(); ++ti) {
-    const TileC& t = B.tilesC_big[ti];
-    int64_t steps = 0;
-    for (int32_t c = t.chunk_begin; c < t.chunk_end; ++c) steps += (pad8(H.chunksC[c].K) + kBigK - 1) / kBigK;
-    const int64_t S = std::max<int64_t>(1, std::min<int64_t>(want, steps / 8));
-    for (int64_t s = 0; s < S; ++s) {
-      B.splitC_tile.push_back((int32_t)ti);
-      B.splitC_begin.push_back((int32_t)(steps * s / S));
-      B.splitC_end.push_back((int32_t)(steps * (s + 1) / S));
-      B.splitC_slot.push_back(S == 1 ? -1 : B.partial_slots + s);
-    }
-    if (S > 1) {
-      B.redC_tile.push_back((int32_t)ti);
-      B.redC_slot.push_back(B.partial_slots);
-      B.redC_nsplit.push_back((int32_t)S);
-      B.partial_slots += S;
-    }
-  }
-  // launch order for the XCDs (see xcd_order): big stage A tiles and big
-  // stage C work items, grouped by 4 x 4 supertiles of their block
+  build_big_items(B.tilesC_big, H.chunksC, kBigTile, kBigK, 2, 32, B.itemsC, B.redsC, B.slotsC);
+  // launch order of the big stage A tiles for the XCDs (see xcd_order), grouped
+  // by 4 x 4 supertiles of their block
   {
     std::unordered_map<int64_t, int64_t> ids;
-    auto key = [&](int64_t problem, int mt, int nt) {
-      const int64_t k = (problem * 8192 + mt / 4) * 8192 + nt / 4;
-      auto it = ids.find(k);
-      if (it == ids.end()) it = ids.emplace(k, (int64_t)ids.size()).first;
-      return it->second;
-    };
     std::vector<int64_t> group, cost;
     for (const TileA16& a : B.tilesA_big) {
-      group.push_back(key(a.c_off, a.mt, a.nt));
+      group.push_back(supertile_key(ids, a.c_off, a.mt, a.nt));
       cost.push_back(a.Kp);
     }
     std::vector<TileA16> outA;
     for (int64_t i : xcd_order(group, cost))
       outA.push_back(i >= 0 ? B.tilesA_big[i] : TileA16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0});
     B.tilesA_big.swap(outA);
-    group.clear();
-    cost.clear();
-    ids.clear();
-    for (size_t w = 0; w < B.splitC_tile.size(); ++w) {
-      const TileC& t = B.tilesC_big[B.splitC_tile[w]];
-      group.push_back(key(t.c_off, t.mt, t.nt));
-      cost.push_back(B.splitC_end[w] - B.splitC_begin[w]);
-    }
-    const int32_t empty = (int32_t)B.tilesC_big.size();  // an empty tile for the padding items
-    std::vector<int32_t> wt, wb, we;
-    std::vector<int64_t> ws;
-    bool padded = false;
-    for (int64_t i : xcd_order(group, cost)) {
-      if (i >= 0) {
-        wt.push_back(B.splitC_tile[i]);
-        wb.push_back(B.splitC_begin[i]);
-        we.push_back(B.splitC_end[i]);
-        ws.push_back(B.splitC_slot[i]);
-      } else {
-        wt.push_back(empty);
-        wb.push_back(0);
-        we.push_back(0);
-        ws.push_back(-1);
-        padded = true;
-      }
-    }
-    if (padded) B.tilesC_big.push_back(TileC{0, 0, 0, 0, 0, 0, 0, 0});
-    B.splitC_tile.swap(wt);
-    B.splitC_begin.swap(wb);
-    B.splitC_end.swap(we);
-    B.splitC_slot.swap(ws);
   }
   for (const ChunkC& c : H.chunksC) {
     ChunkC16 d;

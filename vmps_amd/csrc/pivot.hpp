@@ -292,7 +292,7 @@ struct VConv {             // V block: packed FP64 (K x N, ld K) -> padded split
   int32_t K, N, Kp, pad;
 };
 constexpr int kBigTile = 128;  // workgroup tile edge of the LDS-staged kernels
-constexpr int kBigK = 64;      // k depth of one LDS stage of those kernels
+constexpr int kBigK = 32;      // k depth of a step of the split-BF16 ones
 // A block is handled by the LDS-staged big-tile kernels when both its
 // dimensions are at least this (below, the wave-tile kernels waste less).
 constexpr int kBigMin = 96;
@@ -304,15 +304,9 @@ struct Bf16Layout {
   std::vector<TermC16> comb_terms;
   std::vector<TileA16> tilesA_big;           // 128 x 128 tiles of the large stage A problems
   std::vector<TileC> tilesC_big, tilesC_small;  // stage C tiles: 128-unit and 32-unit
-  // split-K work items of the big stage C tiles: tile index, iteration range
-  // [it_begin, it_end) over the flattened (chunk, 32-deep k block) loop, and
-  // the partial-sum slot (-1 = write the output directly)
-  std::vector<int32_t> splitC_tile, splitC_begin, splitC_end;
-  std::vector<int64_t> splitC_slot;
-  std::vector<int32_t> redC_tile;     // big tiles reduced from partials
-  std::vector<int64_t> redC_slot;     // first partial slot of each reduced tile
-  std::vector<int32_t> redC_nsplit;
-  int64_t partial_slots = 0;          // number of 128 x 128 FP32 partial tiles
+  std::vector<BigItemC> itemsC;  // work items over tilesC_big, in steps of kBigK k
+  std::vector<BigRedC> redsC;    // tiles in several items
+  int64_t slotsC = 0;            // 128 x 128 FP32 partial tiles
   std::vector<TileA16> tilesA;
   std::vector<ChunkC16> chunksC;
   std::vector<TermC16> termsC;
