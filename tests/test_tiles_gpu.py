@@ -166,6 +166,16 @@ def test_lds_tiles_at_block_edges(edge_case, precision, tol, big_min64, xu):
     assert _rel(HxV(H, v), ref) <= tol
 
 
+@pytest.mark.parametrize("precision,tol", [("fp64", FP64_RTOL), ("fp32", 1e-5)])
+@pytest.mark.parametrize("edge", [16, 32])
+def test_wave_tiles_at_block_edges(edge_case, precision, tol, edge):
+    pd, v, ref = edge_case
+    print("wave tiles at edges", precision, edge, flush=True)
+    H = PivotMatrix2(pd, precision=precision)
+    H.set_tiles(wave_edge=edge, big_min64=0, explicit_u=0)
+    assert _rel(HxV(H, v), ref) <= tol
+
+
 @pytest.mark.parametrize("big_min,xu", [(1, 1), (1, 0), (33, 1), (0, 1)])
 def test_bf16x3_tiles_at_block_edges(edge_case, big_min, xu):
     pd, v, ref = edge_case

@@ -54,6 +54,33 @@ struct Mfma<float> {
   __device__ static inline int col(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
+template <class T>
+struct RawLoad;
+template <>
+struct RawLoad<double> {
+  typedef double v2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static double one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
+  }
+  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
+    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b128(r, v, 0, 0));
+  }
+};
+template <>
+struct RawLoad<float> {
+  typedef float v2 __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ static float one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
+  }
+  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
+    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b64(r, v, 0, 0));
+  }
+};
+template <class T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const T* p, int elems) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), (short)0, elems * (int)sizeof(T), 0x00020000);
+}
+
 // A wave computes an E x E output tile (E = 16 or 32) as S x S MFMA
 // accumulators of 16 x 16 (S = E / 16); sub-tiles past the block edge are
 // skipped with wave-uniform tests.
@@ -67,7 +94,7 @@ struct WaveTile {
 #pragma unroll
       for (int y = 0; y < S; ++y) c[x][y] = acc_t{0, 0, 0, 0};
   }
-  // a[x][u]: A[i = m0 + 16x + lane%16][k = 4u + lane/16], b[y][u]: B[k][j = n0 + 16y + lane%16]
+  // a[x][u]: A[i = m0 + 16x + lane%16][k = 4 (lane/16) + u], b[y][u]: B[k][j = n0 + 16y + lane%16]
   __device__ void mac(const T (&a)[S][4], const T (&b)[S][4], bool has_m1, bool has_n1) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -94,6 +121,59 @@ struct WaveTile {
   }
 };
 
+// Operand loads of a wave tile, one 16-deep K block at kb.  Lane group lane/16
+// takes the k's 4 (lane/16) .. + 3, so that B's four are 32 consecutive bytes of
+// its column.  Rows and columns past the block are clamped to its last one
+// (their results are not stored) and the offsets are fixed per lane: the masks
+// and 64-bit addresses of one load per element cost the wave kernels more issue
+// time than their MFMAs (HxV, before and after: FP32 ladder at M = 2048 130 and
+// 90 us, FP64 171 and 141 us, U(1) chain at M = 1024 67 and 51 us, 16 pivots of
+// M <= 1024 211 and 184 us, Hubbard chain at M = 512 21.0 and 20.0 us).
+template <class T, int S>
+struct WaveOff {
+  uint32_t o[S];
+  // A: rows m0 + 16 x + lane%16 of a column-major M x K block
+  __device__ __forceinline__ void rows(int m0, int M, int li, int lk) {
+#pragma unroll
+    for (int x = 0; x < S; ++x) o[x] = (uint32_t)sizeof(T) * (uint32_t)(4 * lk * M + min(m0 + 16 * x + li, M - 1));
+  }
+  // B: columns n0 + 16 y + lane%16 of a column-major K x N block, from column n0 on
+  __device__ __forceinline__ void cols(int n0, int N, int K, int li, int lk) {
+#pragma unroll
+    for (int y = 0; y < S; ++y) o[y] = (uint32_t)sizeof(T) * (uint32_t)(min(16 * y + li, N - 1 - n0) * K + 4 * lk);
+  }
+};
+// past K the buffer's range returns zeros
+template <class T, int S>
+__device__ __forceinline__ void wave_load_a(const T* A, int M, int K, int kb, const WaveOff<T, S>& off, T (&a)[S][4]) {
+  const auto r = raw_buffer(A + (int64_t)kb * M, min(K - kb, 16) * M);
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int x = 0; x < S; ++x) a[x][u] = RawLoad<T>::one(r, off.o[x], (uint32_t)sizeof(T) * (uint32_t)(u * M));
+}
+// B: the block's column n0; lanes past K read past the buffer's end
+template <class T, int S>
+__device__ __forceinline__ void wave_load_b(const T* B, int K, int kb, int lk, const WaveOff<T, S>& off, T (&b)[S][4]) {
+  const auto r = raw_buffer(B + kb, 0x7fffffff / (int)sizeof(T));
+  if (kb + 16 <= K) {
+#pragma unroll
+    for (int y = 0; y < S; ++y) {
+      const auto p = RawLoad<T>::two(r, off.o[y]), q = RawLoad<T>::two(r, off.o[y] + 2 * (uint32_t)sizeof(T));
+      b[y][0] = p[0];
+      b[y][1] = p[1];
+      b[y][2] = q[0];
+      b[y][3] = q[1];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int y = 0; y < S; ++y)
+        b[y][u] = RawLoad<T>::one(r, kb + 4 * lk + u < K ? off.o[y] + u * (uint32_t)sizeof(T) : 0x80000000u, 0);
+  }
+}
+
 // Stage A: T (M x N, ld M) = L (M x K, ld M) . V (K x N, ld K), one E x E tile
 // per wave.  The loads of the next 16-deep K block are issued before the
 // MFMAs of the current one (two register buffers), so a wave waits for memory
@@ -108,25 +188,20 @@ __global__ __launch_bounds__(256) void k_stage_a(const TileA* __restrict__ tiles
   if (w >= ntiles) return;
   const int lane = threadIdx.x & 63;
   const TileA t = tiles[w];
+  if (t.K <= 0) return;  // a padding slot of the launch order (wave-uniform)
   const int m0 = t.mt * E, n0 = t.nt * E;
   const int li = lane & 15, lk = lane >> 4;
   const bool has_m1 = S > 1 && m0 + 16 < t.M, has_n1 = S > 1 && n0 + 16 < t.N;  // wave-uniform
   const T* __restrict__ A = L + t.a_off;
-  const T* __restrict__ B = V + t.b_off;
+  const T* __restrict__ B = V + t.b_off + (int64_t)n0 * t.K;
+  WaveOff<T, S> oa, ob;
+  oa.rows(m0, t.M, li, lk);
+  ob.cols(n0, t.N, t.K, li, lk);
   WaveTile<T, S> acc;
   acc.zero();
-  auto load = [&](int kb, T (&a)[S][4], T (&b)[S][4]) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = kb + 4 * u + lk;
-      const bool kin = k < t.K;
-#pragma unroll
-      for (int x = 0; x < S; ++x) {
-        const int i = m0 + 16 * x + li, j = n0 + 16 * x + li;
-        a[x][u] = (kin && i < t.M) ? A[(int64_t)k * t.M + i] : T(0);
-        b[x][u] = (kin && j < t.N) ? B[(int64_t)j * t.K + k] : T(0);
-      }
-    }
+  auto load = [&](int kb, T (&a)[S][4], T (&b)[S][4]) __attribute__((always_inline)) {
+    wave_load_a<T, S>(A, t.M, t.K, kb, oa, a);
+    wave_load_b<T, S>(B, t.K, kb, lk, ob, b);
   };
   T a0[S][4], b0[S][4], a1[S][4], b1[S][4];
   load(0, a0, b0);
@@ -165,6 +240,8 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
   const bool has_m1 = S > 1 && m0 + 16 < t.M, has_n1 = S > 1 && n0 + 16 < t.N;
   WaveTile<T, S> acc;
   acc.zero();
+  WaveOff<T, S> oa, ob;
+  oa.rows(m0, t.M, li, lk);
   int it = 0;
   for (int g = t.chunk_begin; g < t.chunk_end; g += 64) {
     const int nch = min(64, t.chunk_end - g);
@@ -186,7 +263,8 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
         it += nkb;
         continue;
       }
-      const T* __restrict__ B = R + readlane64(my_r, ci);
+      const T* __restrict__ B = R + readlane64(my_r, ci) + (int64_t)n0 * K;
+      ob.cols(n0, t.N, K, li, lk);
       const int tb = __builtin_amdgcn_readlane(my_tb, ci);
       const int nt = __builtin_amdgcn_readlane(my_te, ci) - tb;
       int64_t my_toff = 0;
@@ -199,54 +277,30 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
       for (int q = first; q < nkb; q += 4) {
         const int kb = q * 16;
         T a[S][4], b[S][4];
+        wave_load_b<T, S>(B, K, kb, lk, ob, b);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = kb + 4 * u + lk;
-          const bool kin = k < K;
-#pragma unroll
-          for (int y = 0; y < S; ++y) {
-            const int j = n0 + 16 * y + li;
-            b[y][u] = (kin && j < t.N) ? B[(int64_t)j * K + k] : T(0);
-          }
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
           for (int x = 0; x < S; ++x) a[x][u] = T(0);
-        }
         int jt = 0;
         for (; jt + 1 < nt; jt += 2) {  // two terms per round, all loads first
-          const T* __restrict__ T0 = Tbuf + readlane64(my_toff, jt);
-          const T* __restrict__ T1 = Tbuf + readlane64(my_toff, jt + 1);
           const T c0 = readlane_t<T>(my_c, jt), c1 = readlane_t<T>(my_c, jt + 1);
           T x0[S][4], x1[S][4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int k = kb + 4 * u + lk;
-            const bool kin = k < K;
-#pragma unroll
-            for (int x = 0; x < S; ++x) {
-              const int i = m0 + 16 * x + li;
-              const bool ok = kin && i < t.M;
-              x0[x][u] = ok ? T0[(int64_t)k * t.M + i] : T(0);
-              x1[x][u] = ok ? T1[(int64_t)k * t.M + i] : T(0);
-            }
-          }
+          wave_load_a<T, S>(Tbuf + readlane64(my_toff, jt), t.M, K, kb, oa, x0);
+          wave_load_a<T, S>(Tbuf + readlane64(my_toff, jt + 1), t.M, K, kb, oa, x1);
 #pragma unroll
           for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int x = 0; x < S; ++x) a[x][u] += c0 * x0[x][u] + c1 * x1[x][u];
         }
         if (jt < nt) {
-          const T* __restrict__ T0 = Tbuf + readlane64(my_toff, jt);
           const T c0 = readlane_t<T>(my_c, jt);
+          T x0[S][4];
+          wave_load_a<T, S>(Tbuf + readlane64(my_toff, jt), t.M, K, kb, oa, x0);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int k = kb + 4 * u + lk;
-            const bool kin = k < K;
+          for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int x = 0; x < S; ++x) {
-              const int i = m0 + 16 * x + li;
-              a[x][u] += c0 * ((kin && i < t.M) ? T0[(int64_t)k * t.M + i] : T(0));
-            }
-          }
+            for (int x = 0; x < S; ++x) a[x][u] += c0 * x0[x][u];
         }
         acc.mac(a, b, has_m1, has_n1);
       }
@@ -294,33 +348,6 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
 //    next slice, the LDS writes of the next step and the loads of the step after
 //    that in between.
 constexpr int kBKd = 16;
-
-template <class T>
-struct RawLoad;
-template <>
-struct RawLoad<double> {
-  typedef double v2 __attribute__((ext_vector_type(2)));
-  __device__ __forceinline__ static double one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
-  }
-  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
-    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b128(r, v, 0, 0));
-  }
-};
-template <>
-struct RawLoad<float> {
-  typedef float v2 __attribute__((ext_vector_type(2)));
-  __device__ __forceinline__ static float one(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
-  }
-  __device__ __forceinline__ static v2 two(__amdgpu_buffer_rsrc_t r, uint32_t v) {
-    return __builtin_bit_cast(v2, __builtin_amdgcn_raw_buffer_load_b64(r, v, 0, 0));
-  }
-};
-template <class T>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const T* p, int elems) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), (short)0, elems * (int)sizeof(T), 0x00020000);
-}
 
 // Staging state of a workgroup: the tile, the operands of the load cursor, and
 // the elements a thread has in flight.
