@@ -666,29 +666,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
 }
 
-// Weighted dot product, pass 1: workgroup b reduces segments [b*spb, (b+1)*spb).
+// Weighted dot product, pass 1: wave w of workgroup b reduces segment 4 b + w
+// (at most 4096 elements), eight loads of each vector in flight per lane.  A
+// segment per wave instead of four per workgroup, one after the other with two
+// loads in flight: 21 -> 10 us on 1.9 M elements in 457 segments.
 __global__ __launch_bounds__(256) void k_dot_partial(const int64_t* __restrict__ seg_off, const int32_t* __restrict__ seg_len,
-                                                     const double* __restrict__ seg_w, int nseg, int spb,
+                                                     const double* __restrict__ seg_w, int nseg,
                                                      const double* __restrict__ x, const double* __restrict__ y,
                                                      double* __restrict__ partial) {
-  __shared__ double red[256];
+  __shared__ double red[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int s = 4 * blockIdx.x + wave;
   double acc = 0.0;
-  const int s0 = blockIdx.x * spb;
-  const int s1 = min(nseg, s0 + spb);
-  for (int s = s0; s < s1; ++s) {
-    const int64_t off = seg_off[s];
+  if (s < nseg) {  // wave-uniform
+    const double* __restrict__ xs = x + seg_off[s];
+    const double* __restrict__ ys = y + seg_off[s];
     const int len = seg_len[s];
-    double part = 0.0;
-    for (int i = threadIdx.x; i < len; i += 256) part += x[off + i] * y[off + i];
-    acc += seg_w[s] * part;
+    int i = lane;
+    for (; i + 7 * 64 < len; i += 8 * 64) {
+      double a[8], b[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        a[u] = xs[i + 64 * u];
+        b[u] = ys[i + 64 * u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += a[u] * b[u];
+    }
+    for (; i < len; i += 64) acc += xs[i] * ys[i];
+    acc *= seg_w[s];
   }
-  red[threadIdx.x] = acc;
+  for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
+  if (lane == 0) red[wave] = acc;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // Pass 2: one workgroup sums the partials in a fixed order.
@@ -726,7 +737,7 @@ __global__ void k_axpy_dev(const double* __restrict__ alpha, double scale, const
   for (; i < n; i += stride) y[i] += a * x[i];
 }
 
-constexpr int kDotSegPerBlock = 4;
+constexpr int kDotSegPerBlock = 4;  // one per wave
 
 inline unsigned grid_for(size_t waves) { return (unsigned)((waves + 3) / 4); }
 
@@ -1025,7 +1036,7 @@ void DevPlan::dot_async(const double* d_x, const double* d_y, double* d_result, 
     return;
   }
   const int nb = (nseg + kDotSegPerBlock - 1) / kDotSegPerBlock;
-  hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(256), 0, s, seg_off.p, seg_len.p, seg_w.p, nseg, kDotSegPerBlock,
+  hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(256), 0, s, seg_off.p, seg_len.p, seg_w.p, nseg,
                      d_x, d_y, partial.p);
   hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, s, partial.p, nb, d_result);
   VMPS_HIP_CHECK(hipGetLastError());

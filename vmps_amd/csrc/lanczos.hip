@@ -41,6 +41,12 @@ __global__ void k_axpby(double a, const double* __restrict__ x, double b, double
   for (; e < n; e += stride) y[e] = a * x[e] + b * y[e];
 }
 
+__global__ void k_fill_zero(double* __restrict__ y, int64_t n) {
+  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (; e < n; e += stride) y[e] = 0.0;
+}
+
 // y = x / sqrt(nrm2[0])
 __global__ void k_normalize_into(const double* __restrict__ nrm2, const double* __restrict__ x, double* __restrict__ y,
                                  int64_t n) {
@@ -75,6 +81,94 @@ __device__ inline double wg_sum(double x) {
   const double r = (ws[0] + ws[1]) + (ws[2] + ws[3]);
   __syncthreads();  // ws is free for the next call
   return r;
+}
+
+// ---- kernels of the correction's conjugate gradients ----------------------------
+// One iteration after q = H' pv: with q0 = q - E pv the projected operator's
+// image is q0 - c psi, c = <psi, q0>, and <pv, image> = <pv, q0> - c <psi, pv>.
+// Three passes read each vector as few times as the dependences allow, and the
+// scalars stay on the device; the host waits once per iteration, for two numbers
+// (five vector updates and three dots with a host round trip each took 170 us
+// beside a 150 us HxV on 1.9 M elements, these 42 us).  Each workgroup sums
+// the kCgParts partial sums of the pass before it, in the same order.
+constexpr int kCgParts = 512;
+
+// sums of n consecutive arrays of kCgParts partials, the same in every workgroup
+template <int n>
+__device__ inline void cg_sums(const double* __restrict__ part, double (&r)[n]) {
+#pragma unroll
+  for (int i = 0; i < n; ++i) {
+    double x = 0.0;
+#pragma unroll
+    for (int u = 0; u < kCgParts / 256; ++u) x += part[i * kCgParts + 256 * u + threadIdx.x];
+    r[i] = wg_sum(x);
+  }
+}
+
+// part[0..2] = <psi, q0>, <pv, q0>, <psi, pv> of workgroup blockIdx.x's elements
+__global__ __launch_bounds__(256) void k_cg_dots(int64_t n, double E, const double* __restrict__ psi,
+                                                 const double* __restrict__ pv, const double* __restrict__ q,
+                                                 const double* __restrict__ ew, double* __restrict__ part) {
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+  const int64_t stride = (int64_t)kCgParts * 256;
+#pragma unroll 4
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += stride) {
+    const double p = pv[e], q0 = q[e] - E * p, wp = ew[e] * psi[e];
+    s0 += wp * q0;
+    s1 += ew[e] * p * q0;
+    s2 += wp * p;
+  }
+  s0 = wg_sum(s0);
+  s1 = wg_sum(s1);
+  s2 = wg_sum(s2);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = s0;
+    part[kCgParts + blockIdx.x] = s1;
+    part[2 * kCgParts + blockIdx.x] = s2;
+  }
+}
+
+// alpha = gg / <pv, image>; t += alpha pv, g -= alpha image, part2 = shares of
+// ||g||^2.  A curvature that is not positive leaves t and g as they are.
+__global__ __launch_bounds__(256) void k_cg_update(int64_t n, double E, const double* __restrict__ part,
+                                                   const double* __restrict__ gg, const double* __restrict__ psi,
+                                                   const double* __restrict__ pv, const double* __restrict__ q,
+                                                   const double* __restrict__ ew, double* __restrict__ t,
+                                                   double* __restrict__ g, double* __restrict__ part2,
+                                                   double* __restrict__ curvature) {
+  double d[3];
+  cg_sums<3>(part, d);
+  const double c = d[0], pq = d[1] - c * d[2];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *curvature = pq;
+  if (!(pq > 0.0)) return;  // uniform over the grid
+  const double alpha = *gg / pq;
+  double s = 0.0;
+  const int64_t stride = (int64_t)kCgParts * 256;
+#pragma unroll 4
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += stride) {
+    const double p = pv[e];
+    t[e] += alpha * p;
+    const double y = g[e] - alpha * (q[e] - E * p - c * psi[e]);
+    g[e] = y;
+    s += ew[e] * y * y;
+  }
+  s = wg_sum(s);
+  if (threadIdx.x == 0) part2[blockIdx.x] = s;
+}
+
+// gg_next = ||g||^2; pv = g + (gg_next / gg) pv
+__global__ __launch_bounds__(256) void k_cg_direction(int64_t n, const double* __restrict__ part2,
+                                                      const double* __restrict__ curvature,
+                                                      const double* __restrict__ gg, const double* __restrict__ g,
+                                                      double* __restrict__ pv, double* __restrict__ gg_next) {
+  if (!(*curvature > 0.0)) return;  // uniform over the grid
+  double d[1];
+  cg_sums<1>(part2, d);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *gg_next = d[0];
+  const double beta = d[0] / *gg;
+  const int64_t stride = (int64_t)kCgParts * 256;
+#pragma unroll 4
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += stride) pv[e] = g[e] + beta * pv[e];
 }
 
 // ---- kernels of the graph-captured iteration ----------------------------------
@@ -879,7 +973,10 @@ RefineResult refine_eigenpair(DevPlan& D, double* d_v, const RefineOpts& o, vmps
   double* t = w + n;   // correction
   double* g = t + n;   // CG residual; -r before the CG
   double* pv = g + n;  // CG direction
-  double* q = pv + n;  // projected operator on pv; H t afterwards
+  double* q = pv + n;  // H' pv; H t afterwards
+  DevBuf<double> cg;   // two values of ||g||^2, the curvature, partial sums
+  cg.alloc(3 + 4 * (size_t)kCgParts);
+  double* cgs = cg.p;
   const vmps_precision saved = D.prec;
   auto apply = [&](vmps_precision p, const double* x, double* y) {
     D.prec = p;
@@ -909,28 +1006,34 @@ RefineResult refine_eigenpair(DevPlan& D, double* d_v, const RefineOpts& o, vmps
       if (res.outer >= o.max_outer || !std::isfinite(rho)) break;
       ++res.outer;
       // CG on the projected correction equation, from t = 0 (residual g = -r);
-      // it stops once the correction reaches half the residual the step needs,
-      // down to 1e-4 of the residual (split-BF16x3 Lanczos vectors, residual
-      // ~3e-4, then reach a 1e-7 residual in one step instead of two)
-      const double cg_tol = std::min(0.1, std::max(o.cg_tol_min, 0.5 * o.tol_state / rho));
-      VMPS_HIP_CHECK(hipMemsetAsync(t, 0, sizeof(double) * n, s));
+      // it stops once the correction reaches a twentieth of the residual the step
+      // needs, down to 1e-4 of the residual (split-BF16x3 Lanczos vectors,
+      // residual ~3e-4, then reach a 1e-7 residual in one step instead of two).
+      // At half, a close second eigenvector could be left in the correction: its
+      // share of the residual is its weight times a small gap, and whether CG
+      // resolved it hung on rounding (U(1) chain at M = 2048, residual 1e-10 asked
+      // for: eigenvectors off by 1e-10 or 6e-9).
+      const double cg_tol = std::min(0.1, std::max(o.cg_tol_min, 0.05 * o.tol_state / rho));
+      hipLaunchKernelGGL(k_fill_zero, dim3(vgrid(n)), dim3(256), 0, s, t, n);
       copy(g, pv);
-      double gg = rho * rho;
+      const double gg0 = rho * rho;
+      VMPS_HIP_CHECK(hipMemcpyAsync(cgs, &gg0, sizeof(double), hipMemcpyHostToDevice, s));
+      VMPS_HIP_CHECK(hipStreamSynchronize(s));  // gg0 is read
       for (int it = 0; it < o.cg_max; ++it) {
+        // ||g||^2 before and after the iteration alternate between two scalars
+        double *gg = cgs + (it & 1), *gg_next = cgs + 1 - (it & 1), *curv = cgs + 2, *part = cgs + 3;
         apply(inner, pv, q);
         ++res.cg_iterations;
-        axpby(-E, pv, 1.0, q);
-        const double c = dot(psi, q);
-        axpby(-c, psi, 1.0, q);
-        const double pq = dot(pv, q);
-        if (!(pq > 0.0)) break;  // not positive definite here: keep the correction so far
-        const double alpha = gg / pq;
-        axpby(alpha, pv, 1.0, t);
-        axpby(-alpha, q, 1.0, g);
-        const double gg_new = dot(g, g);
-        if (std::sqrt(gg_new) <= cg_tol * rho) break;
-        axpby(1.0, g, gg_new / gg, pv);  // pv = g + beta pv
-        gg = gg_new;
+        hipLaunchKernelGGL(k_cg_dots, dim3(kCgParts), dim3(256), 0, s, n, E, psi, pv, q, K.ew.p, part);
+        hipLaunchKernelGGL(k_cg_update, dim3(kCgParts), dim3(256), 0, s, n, E, part, gg, psi, pv, q, K.ew.p, t, g,
+                           part + 3 * kCgParts, curv);
+        hipLaunchKernelGGL(k_cg_direction, dim3(kCgParts), dim3(256), 0, s, n, part + 3 * kCgParts, curv, gg, g, pv,
+                           gg_next);
+        VMPS_HIP_CHECK(hipGetLastError());
+        VMPS_HIP_CHECK(hipMemcpyAsync(K.host3, cgs, 3 * sizeof(double), hipMemcpyDeviceToHost, s));
+        VMPS_HIP_CHECK(hipStreamSynchronize(s));
+        if (!(K.host3[2] > 0.0)) break;  // not positive definite here: keep the correction so far
+        if (std::sqrt(K.host3[1 - (it & 1)]) <= cg_tol * rho) break;
       }
       // t -> unit vector orthogonal to psi
       const double ct = dot(psi, t);
