@@ -279,6 +279,67 @@ __global__ __launch_bounds__(256) void k_sub_combination_dk(const double* __rest
   if (threadIdx.x == 0) norm_part[blockIdx.x] = sum;
 }
 
+// The first pass's subtraction and the second pass's dots for long vectors: w -=
+// sum_{i<=k} c[i] Q_i over the workgroup's 256 elements, then partial[i * nb + b]
+// = sum of ew Q_i w over them, the basis rows kept in LDS between the two, so
+// that a Gram-Schmidt iteration reads the basis three times instead of four
+// (the passes run at HBM rate: 1.9 M elements, 36 rows on average, dots 123 us
+// and subtraction 105 us; the two in one 173 us).  Rows past kSubRows, which two
+// workgroups' LDS per CU cannot hold, are read again, from the cache.
+constexpr int kSubRows = 36;
+__global__ __launch_bounds__(256) void k_sub_dots(const int* __restrict__ kdev, int kofs,
+                                                  const double* __restrict__ Q, int64_t n,
+                                                  const double* __restrict__ c, double* __restrict__ w,
+                                                  const double* __restrict__ ew, double* __restrict__ partial,
+                                                  int nb) {
+  __shared__ double qs[kSubRows][256];
+  __shared__ double ys[256];
+  const int k = *kdev + kofs, tid = threadIdx.x;
+  const int64_t base = (int64_t)blockIdx.x * 256;
+  const int64_t e = min(base + tid, n - 1);  // threads past the end repeat the last element with weight 0
+  double s = 0.0;
+  for (int i = 0; i <= k; i += 16) {
+    double q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = Q[(int64_t)min(i + u, k) * n + e];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (i + u <= k) {  // workgroup-uniform
+        s += c[i + u] * q[u];
+        if (i + u < kSubRows) qs[i + u][tid] = q[u];
+      }
+  }
+  const double y = w[e] - s;
+  __syncthreads();  // no thread reads w[e] after another wrote it
+  if (base + tid < n) w[e] = y;
+  ys[tid] = base + tid < n ? ew[e] * y : 0.0;
+  __syncthreads();
+  const int lane = tid & 63;
+  double wy[4];
+  int64_t at[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    wy[u] = ys[lane + 64 * u];
+    at[u] = min(base + lane + 64 * u, n - 1);
+  }
+  for (int i0 = tid >> 6; i0 <= k; i0 += 16) {  // four rows of this wave per round
+    double acc[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = min(i0 + 4 * r, k);
+      double a = 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a += (i < kSubRows ? qs[i][lane + 64 * u] : Q[(int64_t)i * n + at[u]]) * wy[u];
+      acc[r] = a;
+    }
+    for (int m = 32; m > 0; m >>= 1)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] += __shfl_xor(acc[r], m);
+    if (lane < 4 && i0 + 4 * lane <= k)
+      partial[(int64_t)(i0 + 4 * lane) * nb + blockIdx.x] = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
+  }
+}
+
 // k_multidot_rows_final and k_sub_combination_dk in one kernel, for short
 // partial lists (nb <= kFuseMaxGroups, k < kFuseMaxRows): every workgroup sums
 // the nb partials of each row c[i], i <= k, into LDS (the same sums, in the
@@ -689,17 +750,11 @@ void Krylov::enqueue_iteration(DevPlan& D, hipStream_t s, int kofs) {
   double* c1 = c.p;
   double* c2 = c.p + cap;
   double* c3 = c.p + 2 * cap;
-  auto pass = [&](double* c_out, double* norm_part, int local) {
-    hipLaunchKernelGGL(k_multidot_rows, dim3(ngrp, local ? 1u : gy), dim3(256), 0, s, kdev.p, kofs, Q.p, n, w.p,
-                       ew.p, chunk, gpart.p, ngrp, local);
-    if (fused) {
-      hipLaunchKernelGGL(k_sub_combination_fused, dim3(gs), dim3(256), 0, s, Q.p, n, gpart.p, ngrp, kdev.p, kofs,
-                         c_out, w.p, ew.p, norm_part, local, (const int*)nullptr, 0);
-    } else {
-      hipLaunchKernelGGL(k_multidot_rows_final, dim3(cap), dim3(256), 0, s, kdev.p, kofs, gpart.p, ngrp, c_out);
-      hipLaunchKernelGGL(k_sub_combination_dk, dim3(gs), dim3(256), 0, s, Q.p, n, c_out, kdev.p, kofs, w.p, ew.p,
-                         norm_part);
-    }
+  auto pass = [&](double* c_out, double* norm_part) {
+    hipLaunchKernelGGL(k_multidot_rows, dim3(ngrp, gy), dim3(256), 0, s, kdev.p, kofs, Q.p, n, w.p, ew.p, chunk,
+                       gpart.p, ngrp, 0);
+    hipLaunchKernelGGL(k_sub_combination_fused, dim3(gs), dim3(256), 0, s, Q.p, n, gpart.p, ngrp, kdev.p, kofs,
+                       c_out, w.p, ew.p, norm_part, 0, (const int*)nullptr, 0);
   };
   D.hxv(v.p, w.p, s);
   if (partial_reortho(D)) {
@@ -720,8 +775,19 @@ void Krylov::enqueue_iteration(DevPlan& D, hipStream_t s, int kofs) {
     hipLaunchKernelGGL(k_normalize_next, dim3(gs), dim3(256), 0, s, kdev.p, kofs, npart.p, (int)gs, w.p, Q.p, n,
                        v.p, c1, c2, c3, (const int*)gate.p, out3.p);
   } else {
-    pass(c1, nullptr, 0);
-    pass(c2, npart.p, 0);
+    if (fused) {
+      pass(c1, nullptr);
+      pass(c2, npart.p);
+    } else {
+      const int nsub = (int)((n + 255) / 256);
+      hipLaunchKernelGGL(k_multidot_rows, dim3(ngrp, gy), dim3(256), 0, s, kdev.p, kofs, Q.p, n, w.p, ew.p, chunk,
+                         gpart.p, ngrp, 0);
+      hipLaunchKernelGGL(k_multidot_rows_final, dim3(cap), dim3(256), 0, s, kdev.p, kofs, gpart.p, ngrp, c1);
+      hipLaunchKernelGGL(k_sub_dots, dim3(nsub), dim3(256), 0, s, kdev.p, kofs, Q.p, n, c1, w.p, ew.p, gpart.p, nsub);
+      hipLaunchKernelGGL(k_multidot_rows_final, dim3(cap), dim3(256), 0, s, kdev.p, kofs, gpart.p, nsub, c2);
+      hipLaunchKernelGGL(k_sub_combination_dk, dim3(gs), dim3(256), 0, s, Q.p, n, c2, kdev.p, kofs, w.p, ew.p,
+                         npart.p);
+    }
     hipLaunchKernelGGL(k_normalize_next, dim3(gs), dim3(256), 0, s, kdev.p, kofs, npart.p, (int)gs, w.p, Q.p, n,
                        v.p, c1, c2, (const double*)nullptr, (const int*)nullptr, out3.p);
   }
@@ -1159,7 +1225,9 @@ void Krylov::ensure(DevPlan& D, int kmax) {
   if (n <= (int64_t)kFuseMaxGroups * 8192) ngrp = std::min<int>(ngrp, kFuseMaxGroups);
   chunk = (n + ngrp - 1) / ngrp;
   npart.alloc(vgrid(n));
-  gpart.alloc((size_t)std::max(1, ngrp) * (need + 3));  // rows 0 .. k and k + 1, k + 2 (k_sub_local_dots)
+  // partials of rows 0 .. k and k + 1, k + 2 (k_sub_local_dots), and k_sub_dots' per 256 elements on the long path
+  const bool fused = ngrp <= kFuseMaxGroups && need < kFuseMaxRows;
+  gpart.alloc(std::max((size_t)std::max(1, ngrp) * (need + 3), fused ? 0 : (size_t)((n + 255) / 256) * need));
   VMPS_HIP_CHECK(hipStreamSynchronize(D.stream));
   cap = need;
   nvec = n;
