@@ -209,3 +209,25 @@ def test_lds_tiles_split_k(M, nleft):
     out = HxV(H, v)
     assert _rel(out, ref) <= BF16X3_RTOL
     assert np.array_equal(HxV(H, v), out)
+
+
+def test_bf16x3_wide_tiles_at_block_edges():
+    """Stage C's 128 x 256 split-BF16 tiles (pivots of 256 and more 128 x 128
+    tiles), the last of each block 1 to 4 strips of 32 rows and 64 columns wide,
+    against the FP64 wave tiles."""
+    from vmps_amd import models
+    W = models.heisenberg_u1_mpo()
+    left = [((-1,), 641), ((1,), 700), ((3,), 736), ((5,), 765)]
+    right = [((-1,), 769), ((1,), 595), ((3,), 935), ((5,), 1020)]
+    pd = synth.make_pivot(W, W, left, right, np.random.default_rng(21))
+    v = synth.random_vector(pd, 22)
+    print("wide split-BF16 tiles, vsize", pd.vsize, flush=True)
+    assert pd.vsize >= 256 * 128 * 128
+    H = PivotMatrix2(pd)
+    H.set_tiles(big_min64=0, explicit_u=0)
+    ref = HxV(H, v)
+    H.set_precision("bf16x3")
+    H.set_tiles(big_min=1, explicit_u=1)
+    out = HxV(H, v)
+    assert _rel(out, ref) <= BF16X3_RTOL
+    assert np.array_equal(HxV(H, v), out)

@@ -88,20 +88,20 @@ __global__ __launch_bounds__(256) void k_combine(const CombTask* __restrict__ ta
 
 // Vout tile = sum over its split partials, in slot order; one workgroup per
 // quarter of a tile's columns.
-template <class T, class OutT, int BT>
+template <class T, class OutT, int BT, int BN>
 __global__ __launch_bounds__(256) void k_reduce_big(const TileC* __restrict__ tiles, const BigRedC* __restrict__ reds,
                                                     const T* __restrict__ partial, OutT* __restrict__ Vout) {
   const BigRedC r = reds[blockIdx.x / 4];
   const TileC t = tiles[r.tile];
   const int i = t.mt * BT + threadIdx.x % BT;
   if (i >= t.M) return;
-  const int c0 = (int)(blockIdx.x % 4) * (BT / 4) + threadIdx.x / BT;
-  for (int c = c0; c < (int)(blockIdx.x % 4 + 1) * (BT / 4); c += 256 / BT) {
-    const int j = t.nt * BT + c;
+  const int c0 = (int)(blockIdx.x % 4) * (BN / 4) + threadIdx.x / BT;
+  for (int c = c0; c < (int)(blockIdx.x % 4 + 1) * (BN / 4); c += 256 / BT) {
+    const int j = t.nt * BN + c;
     if (j >= t.N) return;
-    const T* p = partial + r.slot * (int64_t)(BT * BT) + c * BT + threadIdx.x % BT;
+    const T* p = partial + r.slot * (int64_t)(BT * BN) + c * BT + threadIdx.x % BT;
     T acc = p[0];
-    for (int q = 1; q < r.nsplit; ++q) acc += p[(int64_t)q * (BT * BT)];
+    for (int q = 1; q < r.nsplit; ++q) acc += p[(int64_t)q * (BT * BN)];
     Vout[t.c_off + (int64_t)j * t.M + i] = (OutT)acc;
   }
 }

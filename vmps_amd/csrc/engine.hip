@@ -934,7 +934,7 @@ void launch_c_big_edge(DevPlan& D, const T* src, const T* R, double* d_vout, hip
     hipLaunchKernelGGL((k_stage_c_big<T, double, BT, false>), dim3(n), dim3(256), 0, s, D.tilesCb.p, D.itemsCb.p, n,
                        D.chunksC.p, D.termsC.p, src, R, d_vout, part);
   if (nr)
-    hipLaunchKernelGGL((k_reduce_big<T, double, BT>), dim3(4 * nr), dim3(256), 0, s, D.tilesCb.p, D.redsCb.p, part,
+    hipLaunchKernelGGL((k_reduce_big<T, double, BT, BT>), dim3(4 * nr), dim3(256), 0, s, D.tilesCb.p, D.redsCb.p, part,
                        d_vout);
 }
 

@@ -126,6 +126,7 @@ struct DevPlan {
   DevBuf<TileC> bfCsmall, bfCbig;
   DevBuf<BigItemC> itemsC16;  // work items over bfCbig, and the tiles in several of them
   DevBuf<BigRedC> redsC16;
+  bool c16_wide = false;      // bfCbig: 128 x 256 tiles
   DevBuf<float> Cpart;                              // FP32 partial tiles
   DevBuf<ChunkC16> bfC;
   DevBuf<TermC16> bfT;

@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict_
 }
 
 // ---- LDS-staged 128 x 128 workgroup tiles for large blocks -------------------
-// 4 waves in a 2 x 2 grid, sub-blocks of 16 rows and columns dealt to the waves
+// 4 waves in a 2 x 2 grid (8 in a 2 x 4 grid on 128 x 256), sub-blocks of 16 rows and columns dealt to the waves
 // alternately as in the FP64 kernels, and one of 16 instances NX x NY for the
 // tiles at a block's edge.  32-deep K steps, two LDS buffers: while a wave
 // multiplies step i from registers it reads step i + 1's operands from one buffer,
@@ -470,17 +470,28 @@ constexpr int kBT = kBigTile;
 constexpr int kBKs = 32;            // k depth of a step
 constexpr int kLR = 2 * kBKs + 8;   // LDS row: 4 groups of [8 hi | 8 lo], 144 bytes: no bank conflicts
 
-struct BigSmem {  // 72 KB, two workgroups per CU
-  __bf16 A[2][kBT * kLR], B[2][kBT * kLR];
+// NW: waves of the workgroup, and 32-column strips of its tile.  Stage C of pivots
+// with enough tiles takes NW = 8, 128 x 256 tiles: its K loops run hundreds of
+// steps and the workgroups drift apart, so the L2 seldom serves a panel twice, and
+// with 128 columns it fetched 16 GB in 2.8 ms on C60 at M = 4096, more than a
+// copy's rate.  Wider tiles fetch a quarter less; HxV there 6.1 -> 5.4 ms.
+template <int NW>
+struct BigSmem {  // 4 waves: 72 KB, two workgroups per CU; 8 waves: 108 KB
+  __bf16 A[2][kBT * kLR], B[2][32 * NW * kLR];
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t bf_buffer(const __bf16* p, bool on) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p), (short)0, on ? 0x7fffffff : 0, 0x00020000);
 }
 
+template <int NW>
 struct BigTile16 {
-  uint32_t offA[4], offB[4];  // byte offsets of this thread's pieces (rows row + 32 h) at k = 0
-  v8bf ra[4], rb[4];
+  static constexpr int kBN = 32 * NW;   // columns of the tile
+  static constexpr int kCS = 8 * NW;    // columns between a wave's sub-blocks
+  static constexpr int kRS = 8 * NW;    // rows between a thread's pieces
+  static constexpr int kPA = kBT / kRS, kPB = kBN / kRS;
+  uint32_t offA[kPA], offB[kPB];  // byte offsets of this thread's pieces at k = 0
+  v8bf ra[kPA], rb[kPB];
   const __bf16 *A, *B;        // wave-uniform: the tile's first row / column
   int Kp, M, N, m0, n0;
   int row, c8, kk;            // staging role: row, offset in the LDS row, first k of the piece
@@ -492,7 +503,7 @@ struct BigTile16 {
     M = M_;
     N = N_;
     m0 = mt * kBT;
-    n0 = nt * kBT;
+    n0 = nt * kBN;
     li = lane & 15;
     lg = lane >> 4;
     wm = (wave & 1) * 16;
@@ -502,45 +513,45 @@ struct BigTile16 {
     kk = (tid & 6) * 4;
   }
   __device__ __forceinline__ int nx() const { return min(4, (M - m0 + 31) / 32); }  // workgroup-uniform
-  __device__ __forceinline__ int ny() const { return min(4, (N - n0 + 31) / 32); }
+  __device__ __forceinline__ int ny() const { return min(4, (N - n0 + kCS - 1) / kCS); }
   // rows and columns past the block are clamped to its last one (not stored)
   __device__ __forceinline__ void set(const __bf16* Ablk, const __bf16* Bblk, int Kp_) {
     Kp = Kp_;
     A = Ablk + 2 * (int64_t)m0 * Kp;
     B = Bblk + 2 * (int64_t)n0 * Kp;
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      offA[h] = 2u * (uint32_t)(min(row + 32 * h, M - 1 - m0) * 2 * Kp + c8);
-      offB[h] = 2u * (uint32_t)(min(row + 32 * h, N - 1 - n0) * 2 * Kp + c8);
-    }
+    for (int h = 0; h < kPA; ++h) offA[h] = 2u * (uint32_t)(min(row + kRS * h, M - 1 - m0) * 2 * Kp + c8);
+#pragma unroll
+    for (int h = 0; h < kPB; ++h) offB[h] = 2u * (uint32_t)(min(row + kRS * h, N - 1 - n0) * 2 * Kp + c8);
   }
   // K step at kb: pieces at k >= Kp (a multiple of 8) load zeros
   __device__ __forceinline__ void load_a(int kb) {
     const auto r = bf_buffer(A + 2 * kb, kb < Kp);
     const bool in = kb + kk < Kp;
 #pragma unroll
-    for (int h = 0; h < 4; ++h)
+    for (int h = 0; h < kPA; ++h)
       ra[h] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(r, in ? offA[h] : 0x80000000u, 0, 0));
   }
   __device__ __forceinline__ void load_b(int kb) {
     const auto r = bf_buffer(B + 2 * kb, kb < Kp);
     const bool in = kb + kk < Kp;
 #pragma unroll
-    for (int h = 0; h < 4; ++h)
+    for (int h = 0; h < kPB; ++h)
       rb[h] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(r, in ? offB[h] : 0x80000000u, 0, 0));
   }
-  __device__ __forceinline__ void stage_a(BigSmem& s, int buf) const {
+  __device__ __forceinline__ void stage_a(BigSmem<NW>& s, int buf) const {
 #pragma unroll
-    for (int h = 0; h < 4; ++h) st8(&s.A[buf][(row + 32 * h) * kLR + c8], ra[h]);
+    for (int h = 0; h < kPA; ++h) st8(&s.A[buf][(row + kRS * h) * kLR + c8], ra[h]);
   }
-  __device__ __forceinline__ void stage_b(BigSmem& s, int buf) const {
+  __device__ __forceinline__ void stage_b(BigSmem<NW>& s, int buf) const {
 #pragma unroll
-    for (int h = 0; h < 4; ++h) st8(&s.B[buf][(row + 32 * h) * kLR + c8], rb[h]);
+    for (int h = 0; h < kPB; ++h) st8(&s.B[buf][(row + kRS * h) * kLR + c8], rb[h]);
   }
 };
 
-template <int NX, int NY>
+template <int NW, int NX, int NY>
 struct BigAcc16 {
+  typedef BigTile16<NW> Tile;
   v4f acc[NX][NY];
   v8bf a[2][NX][2], b[2][NY][2];  // [step parity][sub-block][hi, lo]
 
@@ -550,13 +561,13 @@ struct BigAcc16 {
 #pragma unroll
       for (int y = 0; y < NY; ++y) acc[x][y] = v4f{0, 0, 0, 0};
   }
-  __device__ __forceinline__ void read(const BigTile16& g, const BigSmem& s, int buf, int p) {
+  __device__ __forceinline__ void read(const Tile& g, const BigSmem<NW>& s, int buf, int p) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
 #pragma unroll
       for (int x = 0; x < NX; ++x) a[p][x][q] = ld8(&s.A[buf][(g.wm + 32 * x + g.li) * kLR + 16 * g.lg + 8 * q]);
 #pragma unroll
-      for (int y = 0; y < NY; ++y) b[p][y][q] = ld8(&s.B[buf][(g.wn + 32 * y + g.li) * kLR + 16 * g.lg + 8 * q]);
+      for (int y = 0; y < NY; ++y) b[p][y][q] = ld8(&s.B[buf][(g.wn + Tile::kCS * y + g.li) * kLR + 16 * g.lg + 8 * q]);
     }
   }
   __device__ __forceinline__ void mac(int p) {  // lo.hi, hi.lo, hi.hi, as mac3 adds them
@@ -570,7 +581,7 @@ struct BigAcc16 {
   }
   // one step from registers p; buffer p ^ 1 holds the next one
   template <class Next>
-  __device__ __forceinline__ void step(BigTile16& g, BigSmem& s, int p, Next&& next) {
+  __device__ __forceinline__ void step(Tile& g, BigSmem<NW>& s, int p, Next&& next) {
     next(g);          // the load cursor moves on
     __syncthreads();  // the next step is staged, and this one's buffer no longer read
     __builtin_amdgcn_sched_barrier(0);
@@ -586,12 +597,12 @@ struct BigAcc16 {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < Tile::kPA + Tile::kPB; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < Tile::kPA + Tile::kPB; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // global load
     }
@@ -599,7 +610,7 @@ struct BigAcc16 {
   }
   // `steps` K steps; next(g) sets the operands and k of the following load (g.kb)
   template <class Next>
-  __device__ __forceinline__ void run(BigTile16& g, BigSmem& s, int steps, Next&& next) {
+  __device__ __forceinline__ void run(Tile& g, BigSmem<NW>& s, int steps, Next&& next) {
     zero();
     if (steps <= 0) return;  // workgroup-uniform
 #pragma unroll
@@ -622,12 +633,12 @@ struct BigAcc16 {
 };
 
 // f(BigAcc16 of the instance covering the tile); workgroup-uniform
-template <class F>
-__device__ __forceinline__ void with_big_acc16(const BigTile16& g, F&& f) {
+template <int NW, class F>
+__device__ __forceinline__ void with_big_acc16(const BigTile16<NW>& g, F&& f) {
   const int nx = g.nx(), ny = g.ny();
 #define VMPS_BIG_ACC(X, Y)     \
   if (nx == X && ny == Y) {    \
-    BigAcc16<X, Y> acc;        \
+    BigAcc16<NW, X, Y> acc;    \
     f(acc);                    \
     return;                    \
   }
@@ -644,17 +655,18 @@ __device__ __forceinline__ void with_big_acc16(const BigTile16& g, F&& f) {
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_a_bf16x3_big(
     const TileA16* __restrict__ tiles, int ntiles, const __bf16* __restrict__ Ls, const __bf16* __restrict__ Vs,
     float* __restrict__ Tp) {
-  __shared__ BigSmem s;
+  __shared__ BigSmem<4> s;
   if ((int)blockIdx.x >= ntiles) return;  // workgroup-uniform
   const TileA16 t = tiles[blockIdx.x];
   if (t.Kp <= 0) return;  // a padding slot of the launch order (workgroup-uniform)
-  BigTile16 g;
+  typedef BigTile16<4> Tile;
+  Tile g;
   g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
   g.set(Ls + 2 * t.a_off, Vs + 2 * t.b_off, t.Kp);
   float* __restrict__ C = Tp + t.c_off;
   with_big_acc16(g, [&](auto& acc) __attribute__((always_inline)) {
     g.kb = -kBKs;
-    acc.run(g, s, (t.Kp + kBKs - 1) / kBKs, [](BigTile16& h) __attribute__((always_inline)) { h.kb += kBKs; });
+    acc.run(g, s, (t.Kp + kBKs - 1) / kBKs, [](Tile& h) __attribute__((always_inline)) { h.kb += kBKs; });
     constexpr int NX = sizeof(acc.acc) / sizeof(acc.acc[0]), NY = sizeof(acc.acc[0]) / sizeof(v4f);
 #pragma unroll
     for (int x = 0; x < NX; ++x) {
@@ -678,22 +690,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 // Stage C, large output blocks: Vout (FP64 col-major M x N) = sum_chunks (sum_j c_j T_j) . R.
 // Work items as in the FP64 kernel (BigItemC, in steps of kBKs k); partial
-// tiles are FP32, column-major 128 x 128.
+// tiles are FP32, column-major, of 128 x 32 NW.
 // kSplitU (explicit stage B): every chunk reads one split block of unit weight
 // from Us, the loads running ahead across the chunks' boundaries; otherwise U
 // is formed and split on the operand load.
-template <bool kSplitU>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_bf16x3_big(
+template <bool kSplitU, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_stage_c_bf16x3_big(
     const TileC* __restrict__ tiles, const BigItemC* __restrict__ items, int nitems,
     const ChunkC16* __restrict__ chunks, const TermC16* __restrict__ terms, const float* __restrict__ Tp,
     const __bf16* __restrict__ Us, const __bf16* __restrict__ Rs, double* __restrict__ Vout,
     float* __restrict__ partial) {
-  __shared__ BigSmem s;
+  typedef BigTile16<NW> Tile;
+  __shared__ BigSmem<NW> s;
   if ((int)blockIdx.x >= nitems) return;  // workgroup-uniform
   const BigItemC w = items[blockIdx.x];
   if (w.tile < 0) return;  // a padding slot of the launch order (workgroup-uniform)
   const TileC t = tiles[w.tile];
-  BigTile16 g;
+  Tile g;
   g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
   int left = w.nsteps, c = w.chunk, kb = w.step * kBKs;
   auto store = [&](auto& acc) __attribute__((always_inline)) {
@@ -706,24 +719,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       for (int y = 0; y < NY; ++y)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int cl = g.wn + 32 * y + 4 * g.lg + v;
+          const int cl = g.wn + Tile::kCS * y + 4 * g.lg + v;
           if (g.n0 + cl >= t.N) continue;
           if (w.slot < 0)
             Vout[t.c_off + (int64_t)(g.n0 + cl) * t.M + g.m0 + r] = (double)acc.acc[x][y][v];
           else
-            partial[w.slot * (int64_t)(kBT * kBT) + cl * kBT + r] = acc.acc[x][y][v];
+            partial[w.slot * (int64_t)(kBT * Tile::kBN) + cl * kBT + r] = acc.acc[x][y][v];
         }
     }
   };
   if constexpr (kSplitU) {
     g.kb = kb - kBKs;
-    auto enter = [&](BigTile16& h) __attribute__((always_inline)) {
+    auto enter = [&](Tile& h) __attribute__((always_inline)) {
       const ChunkC16 ch = chunks[c];
       h.set(Us + 2 * terms[ch.term_begin].t_off, Rs + 2 * ch.r_off, ch.Kp);
     };
     if (left > 0) enter(g);
     with_big_acc16(g, [&](auto& acc) __attribute__((always_inline)) {
-      acc.run(g, s, w.nsteps, [&](BigTile16& h) __attribute__((always_inline)) {
+      acc.run(g, s, w.nsteps, [&](Tile& h) __attribute__((always_inline)) {
         h.kb += kBKs;
         while (h.kb >= h.Kp && left > 0) {
           ++c;
@@ -736,7 +749,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     });
   } else {
     const int lane = threadIdx.x & 63;
-    BigAcc16<4, 4> acc;
+    static_assert(NW == 4, "the fused form stages U with 256 threads");
+    BigAcc16<NW, 4, 4> acc;
     acc.zero();
     const int row = threadIdx.x >> 2, k8 = (threadIdx.x & 3) * 8;  // U pieces: rows row, row + 64, 8 k each
     for (; left > 0; ++c, kb = 0) {
@@ -826,7 +840,9 @@ void DevPlan::upload_bf16_lists(const Bf16Layout& B) {
   bfCbig.upload(B.tilesC_big, stream);
   itemsC16.upload(B.itemsC, stream);
   redsC16.upload(B.redsC, stream);
-  if (Cpart.n < (size_t)(B.slotsC * kBigTile * kBigTile)) Cpart.alloc((size_t)(B.slotsC * kBigTile * kBigTile));
+  c16_wide = B.wideC;
+  const size_t part = (size_t)(B.slotsC * kBigTile * kBigTile * (B.wideC ? 2 : 1));
+  if (Cpart.n < part) Cpart.alloc(part);
   bfC.upload(B.chunksC, stream);
   bfT.upload(B.termsC, stream);
   vconv.upload(B.vconv, stream);
@@ -874,15 +890,21 @@ void DevPlan::launch_stage_bf16x3(int stage, const double* d_vin, double* d_vout
     if (H.explicit_u && bfCombTasks.n)  // stage B: U = sum c T, then stage C reads U
       hipLaunchKernelGGL(k_combine_split, dim3((unsigned)bfCombTasks.n), dim3(256), 0, s, bfCombTasks.p,
                          bfCombTerms.p, Tp.p, (__bf16*)Us.p);
-    if (nW && H.explicit_u)
-      hipLaunchKernelGGL(k_stage_c_bf16x3_big<true>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p, nW,
-                         bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
+    if (nW && c16_wide)
+      hipLaunchKernelGGL((k_stage_c_bf16x3_big<true, 8>), dim3((unsigned)nW), dim3(512), 0, s, bfCbig.p, itemsC16.p,
+                         nW, bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
+    else if (nW && H.explicit_u)
+      hipLaunchKernelGGL((k_stage_c_bf16x3_big<true, 4>), dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p,
+                         nW, bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
     else if (nW)
-      hipLaunchKernelGGL(k_stage_c_bf16x3_big<false>, dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p, nW,
-                         bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
-    if (nR)
-      hipLaunchKernelGGL((k_reduce_big<float, double, kBigTile>), dim3((unsigned)(4 * nR)), dim3(256), 0, s, bfCbig.p,
-                         redsC16.p, Cpart.p, d_vout);
+      hipLaunchKernelGGL((k_stage_c_bf16x3_big<false, 4>), dim3((unsigned)nW), dim3(256), 0, s, bfCbig.p, itemsC16.p,
+                         nW, bfC.p, bfT.p, Tp.p, u, r, d_vout, Cpart.p);
+    if (nR && c16_wide)
+      hipLaunchKernelGGL((k_reduce_big<float, double, kBigTile, 2 * kBigTile>), dim3((unsigned)(4 * nR)), dim3(256), 0,
+                         s, bfCbig.p, redsC16.p, Cpart.p, d_vout);
+    else if (nR)
+      hipLaunchKernelGGL((k_reduce_big<float, double, kBigTile, kBigTile>), dim3((unsigned)(4 * nR)), dim3(256), 0, s,
+                         bfCbig.p, redsC16.p, Cpart.p, d_vout);
     if (nC && H.explicit_u)
       hipLaunchKernelGGL(k_stage_c_bf16x3<true>, dim3((unsigned)nC), dim3(256), 0, s, bfCsmall.p, nC, bfC.p, bfT.p,
                          Tp.p, u, r, d_vout);

@@ -729,11 +729,11 @@ void interleave_queues(const std::vector<std::vector<T>>& queue, const T& paddin
 // of the workgroups resident at once has in all.
 // `kstep`: k depth of a step; `resident`: workgroups per CU; parts keep at least
 // `min_steps` steps, of about 8 microseconds together.
-void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks, int e, int64_t kstep,
+void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks, int e, int en, int64_t kstep,
                      int resident, int64_t min_steps, std::vector<BigItemC>& out, std::vector<BigRedC>& reds,
                      int64_t& slots) {
   constexpr int64_t kCu = 256;
-  const int u = e / 32;
+  const int u = e / 32, cs = std::max(32, en / 4);  // a wave's sub-blocks step 32 rows, cs columns
   reds.clear();
   slots = 0;
   const size_t n = tiles.size();
@@ -742,7 +742,8 @@ void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>&
     const TileC& t = tiles[i];
     for (int32_t c = t.chunk_begin; c < t.chunk_end; ++c) steps[i] += (chunks[c].K + kstep - 1) / kstep;
     // a step's MFMAs in 32 x 32 units, plus its barrier and staging
-    unit[i] = std::min<int64_t>(u, (t.M - t.mt * e + 31) / 32) * std::min<int64_t>(u, (t.N - t.nt * e + 31) / 32) + 1;
+    unit[i] = std::min<int64_t>(u, (t.M - t.mt * e + 31) / 32) *
+                  std::min<int64_t>(en / cs, (t.N - t.nt * en + cs - 1) / cs) + 1;
   }
   // supertiles of 4 x 4 tiles, or fewer while the XCDs would have under 16 each
   std::vector<std::vector<int64_t>> super;
@@ -804,6 +805,14 @@ void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>&
   interleave_queues(items, BigItemC{-1, 0, 0, 0, -1}, out);
 }
 
+// 128 x 128 tiles of stage C's blocks of 128 and more
+int64_t tiles128(const HostPlan& H) {
+  int64_t n = 0;
+  for (const GemmProb& pr : H.probC)
+    if (pr.M >= 128 && pr.N >= 128) n += (int64_t)((pr.M + 127) / 128) * ((pr.N + 127) / 128);
+  return n;
+}
+
 int choose_wave_edge(const HostPlan& H) {
   if (const char* e = std::getenv("VMPS_WAVE_TILE")) {
     const int v = std::atoi(e);
@@ -826,14 +835,11 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
     // their partial sums (FP64, 64 against 128 wide, all problems: C60 at
     // M = 1024 676 / 800 us, U(1) chain at M = 2048 263 / 301 us; C60 at
     // M = 2048 3.73 / 3.56 ms, at M = 4096 25.3 / 23.7 ms).
-    int64_t tiles128 = 0;
-    for (const GemmProb& pr : H.probC)
-      if (pr.M >= 128 && pr.N >= 128) tiles128 += (int64_t)((pr.M + 127) / 128) * ((pr.N + 127) / 128);
-    H.big_edge = tiles128 >= 256 ? 128 : 64;
+    H.big_edge = tiles128(H) >= 256 ? 128 : 64;
     make_tiles(H, H.big_edge, H.crange, H.tilesA_b, H.tilesC_b, big_min64);
     order_for_xcds(H.tilesA_b);
-    build_big_items(H.tilesC_b, H.chunksC, H.big_edge, 16, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b, H.redsC_b,
-                    H.slotsC_b);
+    build_big_items(H.tilesC_b, H.chunksC, H.big_edge, H.big_edge, 16, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b,
+                    H.redsC_b, H.slotsC_b);
   } else {
     H.tilesA_b.clear();
     H.tilesC_b.clear();
@@ -1327,17 +1333,22 @@ void build_bf16_layout(const HostPlan& H, Bf16Layout& B) {
       B.tilesA_big.push_back(a);
     }
   }
+  // 128 x 256 tiles where 128 x 128 ones would give each of the 256 CUs one (the
+  // rule of the FP64 tiles' edge) and U is formed by stage B
+  B.wideC = H.explicit_u && tiles128(H) >= 256;
+  const int wide = B.wideC ? 2 : 1;
   for (const TileC& t : H.tilesC) {
     if (!is_big(t.M, t.N)) {
       B.tilesC_small.push_back(t);
-    } else if (t.mt % (kBigTile / kTile) == 0 && t.nt % (kBigTile / kTile) == 0) {
+    } else if (t.mt % (kBigTile / kTile) == 0 && t.nt % (wide * kBigTile / kTile) == 0) {
       TileC b = t;
       b.mt = (int16_t)(t.mt / (kBigTile / kTile));
-      b.nt = (int16_t)(t.nt / (kBigTile / kTile));
+      b.nt = (int16_t)(t.nt / (wide * kBigTile / kTile));
       B.tilesC_big.push_back(b);
     }
   }
-  build_big_items(B.tilesC_big, H.chunksC, kBigTile, kBigK, 2, 32, B.itemsC, B.redsC, B.slotsC);
+  build_big_items(B.tilesC_big, H.chunksC, kBigTile, wide * kBigTile, kBigK, B.wideC ? 1 : 2, 32, B.itemsC, B.redsC,
+                  B.slotsC);
   // launch order of the big stage A tiles for the XCDs (see xcd_order), grouped
   // by 4 x 4 supertiles of their block
   {

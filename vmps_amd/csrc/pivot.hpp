@@ -306,7 +306,8 @@ struct Bf16Layout {
   std::vector<TileC> tilesC_big, tilesC_small;  // stage C tiles: 128-unit and 32-unit
   std::vector<BigItemC> itemsC;  // work items over tilesC_big, in steps of kBigK k
   std::vector<BigRedC> redsC;    // tiles in several items
-  int64_t slotsC = 0;            // 128 x 128 FP32 partial tiles
+  int64_t slotsC = 0;            // FP32 partial tiles
+  bool wideC = false;            // tilesC_big are 128 x 256 (explicit stage B only)
   std::vector<TileA16> tilesA;
   std::vector<ChunkC16> chunksC;
   std::vector<TermC16> termsC;
