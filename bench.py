@@ -459,7 +459,7 @@ def dmrg_c60_bench(args):
     peak = PEAK_TFLOPS[args.mixed]
     big_tiles = tiles["big_min"] if args.mixed == "bf16x3" else tiles["big_min64"]
     kname = {"A": "k_stage_a", "C": "k_stage_c"}[dom] + ("_bf16x3" if args.mixed == "bf16x3" else "") + \
-        ("_big (128x128 LDS tiles) + small-tile kernel" if big_tiles else "")
+        ("_big (LDS tiles) + small-tile kernel" if big_tiles else "")
     hxv_mixed_ms = ms[3]
     H.close()
     H64 = PivotMatrix2(first_pd, precision="fp64")

@@ -303,7 +303,7 @@ struct Bf16Layout {
   std::vector<CombTask> comb_tasks;          // explicit stage B on the padded layouts
   std::vector<TermC16> comb_terms;
   std::vector<TileA16> tilesA_big;           // 128 x 128 tiles of the large stage A problems
-  std::vector<TileC> tilesC_big, tilesC_small;  // stage C tiles: 128-unit and 32-unit
+  std::vector<TileC> tilesC_big, tilesC_small;  // stage C tiles: 128 x 128 or 256, and 32 x 32
   std::vector<BigItemC> itemsC;  // work items over tilesC_big, in steps of kBigK k
   std::vector<BigRedC> redsC;    // tiles in several items
   int64_t slotsC = 0;            // FP32 partial tiles
