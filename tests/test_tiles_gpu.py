@@ -231,3 +231,27 @@ def test_bf16x3_wide_tiles_at_block_edges():
     out = HxV(H, v)
     assert _rel(out, ref) <= BF16X3_RTOL
     assert np.array_equal(HxV(H, v), out)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", FP64_RTOL), ("bf16x3", BF16X3_RTOL)])
+def test_large_sectors_with_thin_blocks(precision, tol):
+    """A sector of 260 and more does not put every problem on the LDS-staged
+    tiles while the blocks are thin; the tuner's choice gives the same HxV."""
+    from vmps_amd import models
+    W = models.heisenberg_u1_mpo()
+    pd = synth.make_pivot(W, W, [((-1,), 260), ((1,), 5), ((3,), 40)], [((-1,), 3), ((1,), 4), ((3,), 30)],
+                          np.random.default_rng(23))
+    v = synth.random_vector(pd, 24)
+    print("thin blocks", precision, "vsize", pd.vsize, flush=True)
+    lib = oracle.load()
+    h = pivots.build_oracle(lib, pd)
+    try:
+        ref = pivots.oracle_hxv(lib, h, v, nthreads=8)
+    finally:
+        lib.oracle_pivot2_destroy(h)
+    H = PivotMatrix2(pd, precision=precision)
+    cfg = H.tiles()
+    assert cfg["big_min64"] == 128 and cfg["big_min"] == 96 and cfg["explicit_u"] == 1
+    assert _rel(HxV(H, v), ref) <= tol
+    H.autotune(iters=2)
+    assert _rel(HxV(H, v), ref) <= tol

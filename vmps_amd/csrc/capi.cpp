@@ -732,12 +732,12 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
     return (double)ms / iters;
   };
   TileChoice pick{D.H.wave_edge, D.H.big_min, D.H.big_min64, D.H.explicit_u};
-  // Pivots with blocks of 256 and more keep the LDS-staged tiles with the
-  // explicit stage B, which their plans start from, and nothing is left to
-  // time: wave tiles take 1.3 to 2.5 times as long (FP64: C60 at M = 4096 58
+  // Pivots whose large blocks dominate (HostPlan::large) keep the LDS-staged
+  // tiles with the explicit stage B, which their plans start from, and nothing
+  // is left to time: wave tiles take 1.3 to 2.5 times as long (FP64: C60 at M = 4096 58
   // against 24 ms, U(1) chain at M = 2048 339 against 263 us; split-BF16: 174
   // against 96 us there), the fused stage B 1.1 to 1.4 times.
-  const bool large = D.H.stats.max_block_dim >= 2 * vmps::kBigTile;
+  const bool large = D.H.large;
   if (large) {
     pick.explicit_u = true;
     int& threshold = D.prec == VMPS_PREC_BF16X3 ? pick.big_min : pick.big_min64;
@@ -764,9 +764,11 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
       consider(c);
     }
   } else if (!large) {
-    for (int e : {16, 32}) {
+    for (int e : {16, 32}) {  // wave tiles only, U formed on the load
       TileChoice c = pick;
       c.wave_edge = e;
+      c.big_min64 = 0;
+      c.explicit_u = false;
       consider(c);
     }
     TileChoice c = pick;  // every problem on the LDS-staged tiles, U formed once

@@ -813,6 +813,21 @@ int64_t tiles128(const HostPlan& H) {
   return n;
 }
 
+// Stage A's cost on 64 x 64 LDS-staged tiles, in MFMA work: 32 x 32 sub-blocks of
+// 16-deep steps, and as much as one of them for each step's barrier and staging;
+// over the products' own work.  1.25 for full tiles, 1.3 to 1.6 on pivots whose
+// large blocks dominate, 2.5 and more where small ones do.
+double lds_overhead(const HostPlan& H) {
+  double cost = 0, work = 0;
+  for (const GemmProb& p : H.probA) {
+    const double K = H.chunkA[p.chunk_begin].K, steps = std::ceil(K / 16);
+    const int64_t m32 = (p.M + 31) / 32, n32 = (p.N + 31) / 32;
+    cost += steps * (double)(m32 * n32 + ((m32 + 1) / 2) * ((n32 + 1) / 2)) * (16 * 32 * 32);
+    work += K * p.M * p.N;
+  }
+  return work > 0 ? cost / work : 0.0;
+}
+
 int choose_wave_edge(const HostPlan& H) {
   if (const char* e = std::getenv("VMPS_WAVE_TILE")) {
     const int v = std::atoi(e);
@@ -1205,18 +1220,22 @@ void build_plan_tables(const TripleSet& S, HostPlan& H) {
   }
 
   validate_host_plan(H);
-  // Pivots with blocks of 256 and more take the explicit stage B and the
-  // LDS-staged tiles for every problem, in every precision.
-  // For every problem, since a second launch for the small blocks runs on a
-  // nearly empty chip: with blocks below 128 or 32 on wave tiles the U(1) chain at
-  // M = 2048 took 283 or 281 instead of 263 us, C60 at M = 1024 780 or 709
-  // instead of 676 us; split-BF16 with blocks below 96 or all on wave tiles 110
-  // or 151 instead of 96 us and 274 or 358 instead of 242 us (C60 at M = 4096:
-  // 5.6 instead of 5.5 ms for 96).
+  // Pivots with blocks of 256 and more start from the explicit stage B with the
+  // LDS-staged tiles, in every precision, for every problem if large ones
+  // dominate: a second launch for the small blocks then runs on a nearly empty
+  // chip (with blocks below 128 or 32 on wave tiles the U(1) chain at M = 2048
+  // took 283 or 281 instead of 263 us, C60 at M = 1024 780 or 709 instead of
+  // 676 us; split-BF16 with blocks below 96 or all on wave tiles 110 or 151
+  // instead of 96 us and 274 or 358 instead of 242 us; C60 at M = 4096: 5.6
+  // instead of 5.5 ms for 96).  Where small blocks dominate, as in a batch with
+  // one large pivot among many small ones, their tiles would be mostly padding
+  // and barriers (64 pivots of M = 128 to 2048: FP64 5.0 ms against 1.9 on wave
+  // tiles, split-BF16 3.8 against 1.1 ms).
   if (st.max_block_dim >= 2 * kBigTile) {
     H.explicit_u = true;
-    H.big_min = 1;
-    if (H.big_min64 <= 0) H.big_min64 = 1;
+    H.large = lds_overhead(H) < 2.0;
+    if (H.large) H.big_min = 1;
+    if (H.big_min64 <= 0) H.big_min64 = H.large ? 1 : kBigTile;
   }
   build_tiles(H);
   st.n_terms = (int64_t)terms.size();

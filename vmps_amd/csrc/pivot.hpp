@@ -380,6 +380,7 @@ struct HostPlan {
   // LDS-staged tiles tilesA_b / tilesC_b and are absent from the wave
   // lists (0: none do)
   int big_min64 = 0;
+  bool large = false;  // all problems start from, and keep, the LDS-staged tiles (build_plan_tables)
   std::vector<TileA> tilesA_b;
   std::vector<TileC> tilesC_b;
   int big_edge = 128;                 // their edge, 64 or 128
