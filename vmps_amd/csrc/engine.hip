@@ -13,6 +13,7 @@
 // atomics and results are bitwise reproducible run to run.
 #include "engine.hpp"
 #include "combine.hpp"
+#include "tile_loads.hpp"
 #include "wave.hpp"
 
 #include <algorithm>
@@ -347,16 +348,16 @@ __global__ __launch_bounds__(256) void k_stage_c(const TileC* __restrict__ tiles
 //  - a step is scheduled as four slices of NX NY MFMAs with the LDS reads of the
 //    next slice, the LDS writes of the next step and the loads of the step after
 //    that in between.
-constexpr int kBKd = 16;
 
 // Staging state of a workgroup: the tile, the operands of the load cursor, and
 // the elements a thread has in flight.
 template <class T, int BT>
 struct BigTile {
-  static constexpr int S = BT / 32;            // 16 x 16 accumulators per wave and dimension
-  static constexpr int kNA = kBKd * BT / 256;  // A elements per thread and step
-  static constexpr int kNB = kNA / 2;          // B pairs per thread and step
-  static constexpr int kDA = 256 / BT;         // k distance of a thread's A elements
+  typedef BigRole<BT> Role;
+  static constexpr int S = BT / 32;       // 16 x 16 accumulators per wave and dimension
+  static constexpr int kNA = Role::kNA;   // A elements per thread and step
+  static constexpr int kNB = Role::kNB;   // B pairs per thread and step
+  static constexpr int kDA = Role::kDA;   // k distance of a thread's A elements
   // LDS rows start on other banks (64 of 4 bytes) so that neither the reads (16
   // consecutive elements of 4 rows) nor the writes of B's pairs (rows k, k + 2,
   // .. k + 14 of 8 columns) collide: element (k, i) of B at row_b(k) + i
@@ -369,8 +370,8 @@ struct BigTile {
     return k * kRow + (s & (kPad - 1));
   }
   struct Smem {  // FP64, BT = 128: 80 KB, two workgroups fill a CU's 160 KB
-    T A[2][kBKd * kRow];
-    T B[2][kBKd * kRow];
+    T A[2][kBigKd * kRow];
+    T B[2][kBigKd * kRow];
   };
   typedef typename RawLoad<T>::v2 pair_t;
 
@@ -378,8 +379,8 @@ struct BigTile {
   pair_t rb[kNB];
   uint32_t offA, offB[kNB];
   const T *A, *B;      // wave-uniform: k = 0 of the tile's first row / column
-  int M, N, K, m0, n0;
-  int ai, ak, bj, bk;  // staging roles: A row and first k, B column and first k
+  int M, N, K, m0, n0, panelB;
+  Role t;              // staging role
   int wm, wn, li, lk;  // wave's first row / column, lane's row and k
 
   __device__ __forceinline__ void init(int M_, int N_, int mt, int nt, int tid) {
@@ -392,11 +393,8 @@ struct BigTile {
     lk = lane >> 4;
     wm = (wave & 1) * 16;
     wn = (wave >> 1) * 16;
-    ai = tid % BT;
-    ak = tid / BT;
-    bj = tid >> 3;
-    bk = (tid & 7) * 2;
-    offA = (uint32_t)sizeof(T) * (uint32_t)(ak * M + min(ai, M - 1 - m0));
+    t.init(tid);
+    offA = (uint32_t)sizeof(T) * (uint32_t)big_a_first(t.ak, t.ai, M, m0);
   }
   __device__ __forceinline__ int nx() const { return min(S, (M - m0 + 31) / 32); }  // workgroup-uniform
   __device__ __forceinline__ int ny() const { return min(S, (N - n0 + 31) / 32); }
@@ -405,34 +403,35 @@ struct BigTile {
     K = K_;
     A = Ablk + m0;
     B = Bblk + (int64_t)n0 * K;
+    panelB = big_b_panel(BT, N, K, n0, sizeof(T));
 #pragma unroll
     for (int h = 0; h < kNB; ++h)
-      offB[h] = (uint32_t)sizeof(T) * (uint32_t)(min(bj + 32 * h, N - 1 - n0) * K + bk);
+      offB[h] = (uint32_t)sizeof(T) * (uint32_t)big_b_pair(t.bj, h, t.bk, N, K, n0);
   }
-  // K step at kb; nothing is read past K (A by the buffer's range, B by an
-  // offset beyond it), and with kb >= K the loads return zeros
+  // K step at kb: zeros past K (A by the buffer's range, B by an offset beyond
+  // it), and nothing past the block's end
   __device__ __forceinline__ void load_a(int kb) {
-    const auto r = raw_buffer(A + (int64_t)kb * M, max(0, min(K - kb, kBKd) * M - m0));
+    const auto r = raw_buffer(A + (int64_t)kb * M, big_a_range(M, K, kb, m0));
 #pragma unroll
     for (int q = 0; q < kNA; ++q)
-      ra[q] = RawLoad<T>::one(r, offA, (uint32_t)sizeof(T) * (uint32_t)(kDA * q * M));
+      ra[q] = RawLoad<T>::one(r, offA, (uint32_t)sizeof(T) * (uint32_t)big_a_next(kDA, q, M));
   }
   __device__ __forceinline__ void load_b(int kb) {
-    const auto r = raw_buffer(B + kb, kb < K ? 0x7fffffff / (int)sizeof(T) : 0);
-    const bool in0 = kb + bk < K, in1 = kb + bk + 1 < K;
+    const auto r = raw_buffer(B + kb, big_b_range(panelB, K, kb));
+    const bool in0 = big_b_in(kb, t.bk, K), in1 = big_b_in(kb, t.bk + 1, K);
 #pragma unroll
     for (int h = 0; h < kNB; ++h) {
-      rb[h] = RawLoad<T>::two(r, in0 ? offB[h] : 0x80000000u);
+      rb[h] = RawLoad<T>::two(r, in0 ? offB[h] : kNoLoad);
       if (!in1) rb[h][1] = T(0);
     }
   }
   __device__ __forceinline__ void stage(Smem& s, int buf) const {
 #pragma unroll
-    for (int q = 0; q < kNA; ++q) s.A[buf][row_a(ak + kDA * q) + ai] = ra[q];
+    for (int q = 0; q < kNA; ++q) s.A[buf][row_a(t.ak + kDA * q) + t.ai] = ra[q];
 #pragma unroll
     for (int h = 0; h < kNB; ++h) {
-      s.B[buf][row_b(bk) + bj + 32 * h] = rb[h][0];
-      s.B[buf][row_b(bk + 1) + bj + 32 * h] = rb[h][1];
+      s.B[buf][row_b(t.bk) + t.bj + 32 * h] = rb[h][0];
+      s.B[buf][row_b(t.bk + 1) + t.bj + 32 * h] = rb[h][1];
     }
   }
 };
@@ -566,10 +565,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   g.set(L + t.a_off, V + t.b_off, t.K);
   with_big_acc(g, [&](auto& acc) {
     int kb = 0;
-    acc.run(g, s, (t.K + kBKd - 1) / kBKd, [&](BigTile<T, BT>& h) {
+    acc.run(g, s, (t.K + kBigKd - 1) / kBigKd, [&](BigTile<T, BT>& h) {
       h.load_a(kb);
       h.load_b(kb);
-      kb += kBKd;
+      kb += kBigKd;
     });
     acc.store(g, Tout + t.c_off + (int64_t)g.n0 * t.M + g.m0, t.M);
   });
@@ -596,7 +595,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const TileC t = tiles[w.tile];
   Tile g;
   g.init(t.M, t.N, t.mt, t.nt, threadIdx.x);
-  int left = w.nsteps, c = w.chunk, kb = w.step * kBKd;
+  int left = w.nsteps, c = w.chunk, kb = w.step * kBigKd;
   auto out = [&](auto& acc) __attribute__((always_inline)) {
     if (w.slot < 0)
       acc.store(g, Vout + t.c_off + (int64_t)g.n0 * t.M + g.m0, t.M);
@@ -619,7 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         --left;
         h.load_a(kb);
         h.load_b(kb);
-        kb += kBKd;
+        kb += kBigKd;
       });
       out(acc);
     });
@@ -638,7 +637,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         my_c = (T)tm.c;
       }
       g.set(Tbuf, R + ch.r_off, ch.K);
-      for (; kb < ch.K && left > 0; kb += kBKd, --left) {
+      for (; kb < ch.K && left > 0; kb += kBigKd, --left) {
         T u[Tile::kNA];
 #pragma unroll
         for (int q = 0; q < Tile::kNA; ++q) u[q] = T(0);
@@ -656,7 +655,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         g.stage(s, 0);
         __syncthreads();
 #pragma unroll
-        for (int ks = 0; ks < kBKd; ks += 4) {
+        for (int ks = 0; ks < kBigKd; ks += 4) {
           acc.read(g, s, 0, ks, 0);
           acc.mac(0);
         }
