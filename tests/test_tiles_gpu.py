@@ -7,8 +7,8 @@ import numpy as np
 import pytest
 
 import oracle
-from vmps_amd import synth
-from vmps_amd.pivot import HxV, PivotMatrix2, clear_tile_cache
+from vmps_amd import _lib, synth
+from vmps_amd.pivot import DeviceVector, HxV, PivotMatrix2, clear_tile_cache
 
 sys.path.insert(0, __file__.rsplit("/", 1)[0])
 import pivots  # noqa: E402
@@ -255,3 +255,44 @@ def test_large_sectors_with_thin_blocks(precision, tol):
     assert _rel(HxV(H, v), ref) <= tol
     H.autotune(iters=2)
     assert _rel(HxV(H, v), ref) <= tol
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("tiles", [dict(wave_edge=16, big_min64=0, big_min=0, explicit_u=0),
+                                   dict(wave_edge=32, big_min64=0, big_min=0, explicit_u=1),
+                                   dict(big_min64=1, big_min=1, explicit_u=0),
+                                   dict(big_min64=1, big_min=1, explicit_u=1)])
+def test_nan_stays_in_its_blocks(edge_case, precision, tiles):
+    """A vector block of NaN reaches the outputs its terms lead to and no other:
+    an operand's elements past K are zeros, not the memory behind the block (a
+    zero of the other operand would hide finite memory, not NaN).  The other
+    outputs keep every bit; which ones they are, the FP64 product of the block
+    alone says."""
+    pd, v, _ = edge_case
+    print("NaN blocks", precision, tiles, flush=True)
+    probe = PivotMatrix2(pd)
+    H = PivotMatrix2(pd, precision=precision)
+    H.set_tiles(**tiles)
+    din, dout = DeviceVector(H, v), DeviceVector(H)
+
+    def apply(x):
+        din.upload(x)
+        _lib.check(H._lib.vmps_hxv_device(H._plan, din.ptr, dout.ptr, None))
+        return dout.download()
+
+    clean = apply(v)
+    checked = 0
+    for (_, _, _, off, rows, cols) in pd.block_offsets():
+        sl = slice(off, off + rows * cols)
+        alone = np.zeros_like(v)
+        alone[sl] = v[sl]
+        free = HxV(probe, alone) == 0.0
+        x = v.copy()
+        x[sl] = np.nan
+        out = apply(x)
+        assert np.array_equal(out[free], clean[free])
+        assert np.isnan(out).any()
+        checked += int(free.any())
+    assert checked > 10
+    din.free()
+    dout.free()
