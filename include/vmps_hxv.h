@@ -229,8 +229,9 @@ vmps_status vmps_plan_time_hxv(vmps_plan* plan, int warmup, int iters, double* m
  * GEMMs need none); it serves the GPU path's tuning.
  *   wave_edge: output tile edge of the FP64 / FP32 wave kernels, 16 or 32;
  *   big_min:   split-BF16 x3 only: problems with both dimensions >= big_min
- *              use the LDS-staged 128 x 128 workgroup tiles, the rest
- *              32 x 32 wave tiles (0 = none use the big tiles);
+ *              use the LDS-staged workgroup tiles (128 x 128, stage C of
+ *              pivots with enough of them 128 x 256), the rest 32 x 32 wave
+ *              tiles (0 = none use the LDS-staged ones);
  *   big_min64: FP64 / FP32 only: problems with both dimensions >= big_min64
  *              use LDS-staged 64 x 64 or 128 x 128 workgroup tiles (0 = none);
  *   explicit_u: 0 = the combine U = sum c T is done on stage C's operand

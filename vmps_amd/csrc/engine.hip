@@ -13,7 +13,6 @@
 // atomics and results are bitwise reproducible run to run.
 #include "engine.hpp"
 #include "combine.hpp"
-#include "tile_loads.hpp"
 #include "wave.hpp"
 
 #include <algorithm>

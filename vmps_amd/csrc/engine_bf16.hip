@@ -467,7 +467,8 @@ __global__ __launch_bounds__(256) void k_stage_c_bf16x3(const TileC* __restrict_
 // whole 128-byte lines.  (A single-buffered 64-deep form with masked loads and
 // separate arrays: 278.)
 constexpr int kBT = kBigTile;
-constexpr int kBKs = 32;            // k depth of a step
+constexpr int kBKs = kBigK;         // k depth of a step, in which the work items count
+static_assert(kBKs == 32, "a row of a step is 8 pieces of 16 bytes, one per thread");
 constexpr int kLR = 2 * kBKs + 8;   // LDS row: 4 groups of [8 hi | 8 lo], 144 bytes: no bank conflicts
 
 // NW: waves of the workgroup, and 32-column strips of its tile.  Stage C of pivots

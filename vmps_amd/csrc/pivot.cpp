@@ -814,15 +814,15 @@ int64_t tiles128(const HostPlan& H) {
 }
 
 // Stage A's cost on 64 x 64 LDS-staged tiles, in MFMA work: 32 x 32 sub-blocks of
-// 16-deep steps, and as much as one of them for each step's barrier and staging;
+// kBigKd-deep steps, and as much as one of them for each step's barrier and staging;
 // over the products' own work.  1.25 for full tiles, 1.3 to 1.6 on pivots whose
 // large blocks dominate, 2.5 and more where small ones do.
 double lds_overhead(const HostPlan& H) {
   double cost = 0, work = 0;
   for (const GemmProb& p : H.probA) {
-    const double K = H.chunkA[p.chunk_begin].K, steps = std::ceil(K / 16);
+    const double K = H.chunkA[p.chunk_begin].K, steps = std::ceil(K / kBigKd);
     const int64_t m32 = (p.M + 31) / 32, n32 = (p.N + 31) / 32;
-    cost += steps * (double)(m32 * n32 + ((m32 + 1) / 2) * ((n32 + 1) / 2)) * (16 * 32 * 32);
+    cost += steps * (double)(m32 * n32 + ((m32 + 1) / 2) * ((n32 + 1) / 2)) * (kBigKd * 32 * 32);
     work += K * p.M * p.N;
   }
   return work > 0 ? cost / work : 0.0;
@@ -853,7 +853,7 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
     H.big_edge = tiles128(H) >= 256 ? 128 : 64;
     make_tiles(H, H.big_edge, H.crange, H.tilesA_b, H.tilesC_b, big_min64);
     order_for_xcds(H.tilesA_b);
-    build_big_items(H.tilesC_b, H.chunksC, H.big_edge, H.big_edge, 16, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b,
+    build_big_items(H.tilesC_b, H.chunksC, H.big_edge, H.big_edge, kBigKd, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b,
                     H.redsC_b, H.slotsC_b);
   } else {
     H.tilesA_b.clear();

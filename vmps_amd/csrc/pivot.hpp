@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "sym.hpp"
+#include "tile_loads.hpp"
 
 namespace vmps {
 
@@ -228,10 +229,11 @@ struct TileC {             // Vout(M x N, ld M) tile = sum over chunks U . R
   int16_t mt, nt;
   int32_t pad;
 };
-// LDS-staged FP64 / FP32 tiles of stage C: K steps [step, step + nsteps) of the
-// tile's flattened (chunk, 16-deep K step) sequence, counted from `step` of
-// chunk `chunk`.  slot < 0: the item is the whole tile and writes the output;
-// else it writes partial tile `slot`.
+// Work item of an LDS-staged tile of stage C: nsteps steps of the tile's flattened
+// (chunk, K step) sequence, from step `step` of chunk `chunk` on.  A step is kBigKd
+// deep on the FP64 / FP32 tiles and kBigK deep on the split-BF16 ones.  slot < 0:
+// the item is the whole tile and writes the output; else it writes partial tile
+// `slot`.
 struct BigItemC {
   int32_t tile, chunk, step, nsteps;  // tile < 0: padding of the launch order
   int64_t slot;
@@ -291,7 +293,7 @@ struct VConv {             // V block: packed FP64 (K x N, ld K) -> padded split
   int64_t src_off, dst_off;
   int32_t K, N, Kp, pad;
 };
-constexpr int kBigTile = 128;  // workgroup tile edge of the LDS-staged kernels
+constexpr int kBigTile = 128;  // workgroup tile edge of the split-BF16 LDS-staged kernels, of FP64 / FP32 at most
 constexpr int kBigK = 32;      // k depth of a step of the split-BF16 ones
 // A block is handled by the LDS-staged big-tile kernels when both its
 // dimensions are at least this (below, the wave-tile kernels waste less).

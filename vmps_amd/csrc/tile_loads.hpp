@@ -17,7 +17,7 @@
 
 namespace vmps {
 
-constexpr int kBigKd = 16;                      // k depth of a step
+constexpr int kBigKd = 16;                      // k depth of a step (work items count in it too)
 constexpr uint32_t kNoLoad = 0x80000000u;       // a byte offset past every range
 constexpr int64_t kMaxRangeBytes = 0x7fffffff;  // of a buffer descriptor
 
