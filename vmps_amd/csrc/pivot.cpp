@@ -805,6 +805,56 @@ void build_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>&
   interleave_queues(items, BigItemC{-1, 0, 0, 0, -1}, out);
 }
 
+}  // namespace
+
+void check_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks, int64_t kstep,
+                     const std::vector<BigItemC>& items, const std::vector<BigRedC>& reds, int64_t slots) {
+  auto need = [](bool ok, const char* what) {
+    if (!ok) throw VmpsError(VMPS_ERR_INTERNAL, std::string("stage C work items: ") + what);
+  };
+  std::vector<int64_t> at(chunks.size() + 1, 0);  // K steps before each chunk
+  for (size_t c = 0; c < chunks.size(); ++c) at[c + 1] = at[c] + (chunks[c].K + kstep - 1) / kstep;
+  std::vector<int64_t> done(tiles.size(), 0);
+  std::vector<int32_t> count(tiles.size(), 0), owner((size_t)std::max<int64_t>(0, slots), -1);
+  for (const BigItemC& w : items) {
+    if (w.tile < 0) continue;  // padding of the launch order
+    need(w.tile < (int64_t)tiles.size(), "tile out of range");
+    const TileC& t = tiles[w.tile];
+    need(t.chunk_begin >= 0 && t.chunk_begin <= t.chunk_end && t.chunk_end <= (int64_t)chunks.size(),
+         "chunks of a tile out of range");
+    const int64_t total = at[t.chunk_end] - at[t.chunk_begin];
+    need(w.nsteps >= 0 && done[w.tile] + w.nsteps <= total, "more steps than the tile has");
+    if (w.nsteps > 0) {
+      need(w.chunk >= t.chunk_begin && w.chunk < t.chunk_end, "chunk out of range");
+      need(w.step >= 0 && w.step < at[w.chunk + 1] - at[w.chunk], "step out of range");
+      need(at[w.chunk] + w.step - at[t.chunk_begin] == done[w.tile], "steps missing or taken twice");
+    }
+    done[w.tile] += w.nsteps;
+    ++count[w.tile];
+    if (w.slot < 0) {
+      need(w.nsteps == total, "part of a tile without a slot");
+    } else {
+      need(w.slot < slots && owner[w.slot] < 0, "slot out of range or taken twice");
+      owner[w.slot] = w.tile;
+    }
+  }
+  std::vector<int32_t> parts(tiles.size(), 0);
+  for (const BigRedC& r : reds) {
+    need(r.tile >= 0 && r.tile < (int64_t)tiles.size() && r.nsplit > 0 && r.slot >= 0 && r.slot + r.nsplit <= slots,
+         "reduction out of range");
+    for (int32_t q = 0; q < r.nsplit; ++q) need(owner[r.slot + q] == r.tile, "reduction of another tile's parts");
+    need(parts[r.tile] == 0, "tile reduced twice");
+    parts[r.tile] = r.nsplit;
+  }
+  for (const BigItemC& w : items)
+    if (w.tile >= 0)
+      need(w.slot < 0 ? count[w.tile] == 1 && parts[w.tile] == 0 : parts[w.tile] == count[w.tile],
+           "parts of a tile not reduced");
+  for (size_t i = 0; i < tiles.size(); ++i)
+    need(count[i] > 0 && done[i] == at[tiles[i].chunk_end] - at[tiles[i].chunk_begin], "tile not covered");
+}
+
+namespace {
 // 128 x 128 tiles of stage C's blocks of 128 and more
 int64_t tiles128(const HostPlan& H) {
   int64_t n = 0;
@@ -855,6 +905,7 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
     order_for_xcds(H.tilesA_b);
     build_big_items(H.tilesC_b, H.chunksC, H.big_edge, H.big_edge, kBigKd, H.big_edge == 64 ? 3 : 2, 16, H.itemsC_b,
                     H.redsC_b, H.slotsC_b);
+    check_big_items(H.tilesC_b, H.chunksC, kBigKd, H.itemsC_b, H.redsC_b, H.slotsC_b);
   } else {
     H.tilesA_b.clear();
     H.tilesC_b.clear();
@@ -1368,6 +1419,7 @@ void build_bf16_layout(const HostPlan& H, Bf16Layout& B) {
   }
   build_big_items(B.tilesC_big, H.chunksC, kBigTile, wide * kBigTile, kBigK, B.wideC ? 1 : 2, 32, B.itemsC, B.redsC,
                   B.slotsC);
+  check_big_items(B.tilesC_big, H.chunksC, kBigK, B.itemsC, B.redsC, B.slotsC);
   // launch order of the big stage A tiles for the XCDs (see xcd_order), grouped
   // by 4 x 4 supertiles of their block
   {

@@ -460,5 +460,10 @@ std::string tile_signature(const HostPlan& H);
 void build_bf16_layout(const HostPlan& H, Bf16Layout& B);
 // Throws VMPS_ERR_INTERNAL if any descriptor would address outside its buffer.
 void validate_host_plan(const HostPlan& H);
+// ... if the work items of LDS-staged stage C tiles, in steps of kstep k, do not cover
+// every K step of every tile once and in order, inside its chunks, or if a
+// partial tile's slot is out of range, shared, or not summed into its tile.
+void check_big_items(const std::vector<TileC>& tiles, const std::vector<ChunkC>& chunks, int64_t kstep,
+                     const std::vector<BigItemC>& items, const std::vector<BigRedC>& reds, int64_t slots);
 
 }  // namespace vmps
