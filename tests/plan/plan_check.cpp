@@ -112,7 +112,18 @@ static void corrupt(const Lists& good) {
   refused("reduction past the slots", [&](Lists& b) { b.reds.back().slot = b.slots; return true; });
 }
 
+// one large block row against a thin one: the same classes and work in the
+// histogram, but only the first is dominated by large blocks
+static void signatures() {
+  HostPlan a, b;
+  build_plan(triples({320}, {64}), a);
+  build_plan(triples({400}, {33}), b);
+  expect(a.large && !b.large, "one plan of each kind");
+  expect(tile_signature(a) != tile_signature(b), "plans of different rules have different signatures");
+}
+
 int main() {
+  signatures();
   std::mt19937 rng(5);
   int split = 0, edge128 = 0, wide = 0;
   const std::vector<std::vector<int64_t>> bonds = {{1, 17, 64, 65, 130}, {3, 260, 31, 127}, {300, 5, 257}, {640, 29},

@@ -1,6 +1,7 @@
 """Work lists of the LDS-staged stage C tiles: those the library builds cover
 every K step of every tile once, and a wrong entry is refused before it reaches
-the device (tests/plan/plan_check.cpp, against the built library)."""
+the device; a plan's tuning key tells plans of different rules apart
+(tests/plan/plan_check.cpp, against the built library)."""
 import os
 import subprocess
 
@@ -16,6 +17,6 @@ def build(name, tmp_path):
     return exe
 
 
-def test_work_items_are_checked(tmp_path):
+def test_work_items_and_signatures(tmp_path):
     r = subprocess.run([build("plan_check", tmp_path)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -967,6 +967,8 @@ std::string tile_signature(const HostPlan& H) {
       }
   // the total work decides whether launches or MFMA time dominate
   key += "w" + std::to_string(total > 0 ? (int)std::floor(std::log2(total)) : 0);
+  // plans dominated by large blocks are tuned by another rule (vmps_plan_autotune)
+  if (H.large) key += "L";
   return key;
 }
 
