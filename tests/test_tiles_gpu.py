@@ -296,3 +296,29 @@ def test_nan_stays_in_its_blocks(edge_case, precision, tiles):
     assert checked > 10
     din.free()
     dout.free()
+
+
+def _large_pivot():
+    from vmps_amd import models
+    W = models.heisenberg_u1_mpo()
+    return synth.make_pivot(W, W, [((-1,), 300), ((1,), 280)], [((-1,), 290), ((1,), 257)], np.random.default_rng(41))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+def test_autotune_of_a_large_pivot_drops_hand_set_tiles(precision):
+    """A pivot dominated by large blocks is tuned among its rule's own choices: a
+    slow configuration set by hand before is neither kept nor cached, and the
+    other precisions' threshold does not travel with the choice."""
+    pd = _large_pivot()
+    print("hand-set tiles, then autotune", precision, flush=True)
+    clear_tile_cache()
+    H = PivotMatrix2(pd, precision=precision)
+    assert H.tiles()["big_min"] == 1 and H.tiles()["big_min64"] == 1
+    H.set_tiles(big_min=512, big_min64=512, explicit_u=0)
+    cfg = H.autotune(iters=1)
+    used = "big_min" if precision == "bf16x3" else "big_min64"
+    assert cfg[used] in (0, 1) and cfg["explicit_u"] == 1
+    H2 = PivotMatrix2(pd, precision=precision)
+    cfg2 = H2.autotune(iters=1)
+    assert cfg2["from_cache"] == 1 and cfg2[used] == cfg[used] and cfg2["explicit_u"] == 1
+    assert cfg2["big_min64" if precision == "bf16x3" else "big_min"] == 1

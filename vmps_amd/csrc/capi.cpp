@@ -703,6 +703,7 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
   require(plan && iters > 0, VMPS_ERR_ARG, "bad argument");
   auto& D = plan->D;
   const std::string key = std::to_string((int)D.prec) + "/" + vmps::tile_signature(D.H);
+  const bool bf16 = D.prec == VMPS_PREC_BF16X3;
   auto result = [&](double ms, int from_cache, int tried) {
     return vmps_tile_config{D.H.wave_edge, D.H.big_min, D.H.big_min64, D.H.explicit_u ? 1 : 0, ms, from_cache, tried};
   };
@@ -710,16 +711,19 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     auto it = g_tune_cache.find(key);
     if (it != g_tune_cache.end()) {
-      D.retile(it->second.wave_edge, it->second.big_min, it->second.big_min64, it->second.explicit_u);
+      const TileChoice& c = it->second;  // the parameters that another precision uses stay as they are
+      if (bf16)
+        D.retile(D.H.wave_edge, c.big_min, D.H.big_min64, c.explicit_u);
+      else
+        D.retile(c.wave_edge, D.H.big_min, c.big_min64, c.explicit_u);
       if (out) *out = result(0.0, 1, 0);
       return VMPS_OK;
     }
   }
-  // Coordinate search from the plan's current configuration over the
-  // parameters its precision uses (the others stay as they are): each
-  // parameter's other values in turn, keeping the best so far.  Four
-  // candidates instead of the eight (FP64 / FP32) or six (split-BF16) of the
-  // full grid; one warm-up call per candidate absorbs its first-call set-up.
+  // Search from the plan's current configuration over the parameters its
+  // precision uses (the others stay as they are), keeping the best so far: at
+  // most six candidates; one warm-up call per candidate absorbs its first-call
+  // set-up.
   auto measure = [&](const TileChoice& c) {
     D.retile(c.wave_edge, c.big_min, c.big_min64, c.explicit_u);
     D.hxv(D.vin.p, D.vout.p, D.stream);
@@ -737,11 +741,12 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
   // is left to time: wave tiles take 1.3 to 2.5 times as long (FP64: C60 at M = 4096 58
   // against 24 ms, U(1) chain at M = 2048 339 against 263 us; split-BF16: 174
   // against 96 us there), the fused stage B 1.1 to 1.4 times.
+  // A configuration set by hand before is no candidate: it would reach later
+  // plans through the cache without having been compared with anything.
   const bool large = D.H.large;
   if (large) {
     pick.explicit_u = true;
-    int& threshold = D.prec == VMPS_PREC_BF16X3 ? pick.big_min : pick.big_min64;
-    if (threshold <= 0) threshold = 1;
+    (bf16 ? pick.big_min : pick.big_min64) = 1;
   }
   double best = measure(pick);
   int tried = 1;
@@ -756,7 +761,7 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
       pick = c;
     }
   };
-  if (!large && D.prec == VMPS_PREC_BF16X3) {
+  if (!large && bf16) {
     const TileChoice base = pick;
     for (int b : {vmps::kBigMin, 2 * vmps::kBigMin, 0}) {
       TileChoice c = base;
