@@ -738,9 +738,20 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
   TileChoice pick{D.H.wave_edge, D.H.big_min, D.H.big_min64, D.H.explicit_u};
   // Pivots whose large blocks dominate (HostPlan::large) keep the LDS-staged
   // tiles with the explicit stage B, which their plans start from, and nothing
-  // is left to time: wave tiles take 1.3 to 2.5 times as long (FP64: C60 at M = 4096 58
-  // against 24 ms, U(1) chain at M = 2048 339 against 263 us; split-BF16: 174
-  // against 96 us there), the fused stage B 1.1 to 1.4 times.
+  // is timed.  LDS-staged against wave tiles, stage B explicit in both:
+  //  - three plans in flight on their own streams, us, FP64 and FP32: U(1) chain at
+  //    M = 1500 113 / 114 and 62 / 68, at M = 2048 226 / 232 and 127 / 140; C60 at M = 1024
+  //    608 / 665 and 343 / 414;
+  //  - one plan, its calls back to back: 146 / 132 and 102 / 91, 269 / 238 and 173 /
+  //    149, 690 / 680 and 414 / 381 there (the LDS-staged tiles' last round leaves CUs
+  //    idle); C60 at M = 2048 3574 / 3881 and 2137 / 2409, at M = 4096 23.7 / 36.0 and
+  //    13.3 / 24.9 ms;
+  //  - split-BF16, back to back: 72 / 82, 97 / 151, 235 / 356, 1000 / 2580 us up to C60
+  //    at M = 2048.
+  // The fused stage B takes 1.01 to 1.35 times as long (split-BF16: 1.2 to 1.5).  The
+  // tuner times one plan back to back, so on the smallest of these pivots it
+  // would choose what is slower beside other work; a program whose pivots are
+  // alone on the card can set the wave tiles by hand.
   // A configuration set by hand before is no candidate: it would reach later
   // plans through the cache without having been compared with anything.
   const bool large = D.H.large;

@@ -897,7 +897,7 @@ void set_wave_edge(HostPlan& H, int edge, int big_min64) {
     make_tiles(H, edge, H.crange, H.tilesA_w, H.tilesC_w, -big_min64);
     // 128 x 128 tiles once stage C's blocks of 128 and more give each of the 256 CUs one:
     // below that the K loops would have to be cut into parts too short for
-    // their partial sums (FP64, 64 against 128 wide, all problems: C60 at
+    // their partial sums (FP64, one plan, its calls back to back, 64 against 128 wide, all problems: C60 at
     // M = 1024 676 / 800 us, U(1) chain at M = 2048 263 / 301 us; C60 at
     // M = 2048 3.73 / 3.56 ms, at M = 4096 25.3 / 23.7 ms).
     H.big_edge = tiles128(H) >= 256 ? 128 : 64;
@@ -1276,8 +1276,8 @@ void build_plan_tables(const TripleSet& S, HostPlan& H) {
   // Pivots with blocks of 256 and more start from the explicit stage B with the
   // LDS-staged tiles, in every precision, for every problem if large ones
   // dominate: a second launch for the small blocks then runs on a nearly empty
-  // chip (with blocks below 128 or 32 on wave tiles the U(1) chain at M = 2048
-  // took 283 or 281 instead of 263 us, C60 at M = 1024 780 or 709 instead of
+  // chip (FP64, one plan, its calls back to back: with blocks below 128 or 32 on wave
+  // tiles the U(1) chain at M = 2048 took 277 or 281 instead of 263 us, C60 at M = 1024 780 or 709 instead of
   // 676 us; split-BF16 with blocks below 96 or all on wave tiles 110 or 151
   // instead of 96 us and 274 or 358 instead of 242 us; C60 at M = 4096: 5.6
   // instead of 5.5 ms for 96).  Where small blocks dominate, as in a batch with
