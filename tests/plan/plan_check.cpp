@@ -122,8 +122,32 @@ static void signatures() {
   expect(tile_signature(a) != tile_signature(b), "plans of different rules have different signatures");
 }
 
+// the widths of the LDS tiles change at 256 tiles of 128 x 128 in blocks of 128 and more
+static void widths() {
+  for (int64_t n : {255, 256}) {
+    HostPlan H;
+    build_plan(triples({128}, {128 * n}), H);
+    expect(H.big_min64 > 0 && H.big_edge == (n < 256 ? 64 : 128), "edge of the FP64 / FP32 tiles");
+    for (bool xu : {false, true}) {
+      H.explicit_u = xu;
+      build_tiles(H);
+      Bf16Layout B;
+      build_bf16_layout(H, B);
+      expect(B.wideC == (xu && n >= 256), "width of the split-BF16 stage C tiles");
+    }
+  }
+  // a pivot of the size that the 128-wide kernels are tested with: tiles cut along K
+  HostPlan H;
+  build_plan(triples({641, 700, 736, 765}, {769, 595, 935, 1020}), H);
+  Bf16Layout B;
+  build_bf16_layout(H, B);
+  expect(H.big_edge == 128 && !H.redsC_b.empty(), "128-wide tiles cut along K");
+  expect(B.wideC && !B.redsC.empty(), "128 x 256 tiles cut along K");
+}
+
 int main() {
   signatures();
+  widths();
   std::mt19937 rng(5);
   int split = 0, edge128 = 0, wide = 0;
   const std::vector<std::vector<int64_t>> bonds = {{1, 17, 64, 65, 130}, {3, 260, 31, 127}, {300, 5, 257}, {640, 29},

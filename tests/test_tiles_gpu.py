@@ -124,9 +124,9 @@ def test_set_tiles_rejects_bad_edge(case):
 @pytest.mark.parametrize("precision,tol", [("fp64", FP64_RTOL), ("fp32", 1e-5)])
 @pytest.mark.parametrize("big_min64,xu", [(96, 0), (64, 1), (128, 1)])
 def test_fp64_fp32_big_tiles(case, precision, tol, big_min64, xu):
-    """LDS-staged 128 x 128 FP64 / FP32 tiles for the problems >= big_min64
-    (with the fused and with the explicit stage B) against the oracle; FP64 is
-    bit-identical to the wave tiles only up to summation order."""
+    """LDS-staged FP64 / FP32 tiles, 64 wide on a pivot of this size, for the
+    problems >= big_min64 (with the fused and with the explicit stage B) against the
+    oracle; FP64 is bit-identical to the wave tiles only up to summation order."""
     pd, v, ref = case
     print("big tiles", precision, big_min64, xu, flush=True)
     H = PivotMatrix2(pd, precision=precision)
@@ -185,10 +185,17 @@ def test_bf16x3_tiles_at_block_edges(edge_case, big_min, xu):
     assert _rel(HxV(H, v), ref) <= BF16X3_RTOL
 
 
+def _tiles128(pd):
+    """128 x 128 tiles of the vector's blocks of 128 and more.  From 256 on the FP64
+    and FP32 LDS tiles are 128 wide instead of 64, and split-BF16 stage C's 128 x 256
+    with the explicit stage B (the rule itself: tests/plan/plan_check.cpp)."""
+    return sum(-(-r // 128) * -(-c // 128) for (_, _, _, _, r, c) in pd.block_offsets() if min(r, c) >= 128)
+
+
 @pytest.mark.parametrize("M,nleft", [(640, 29), (2047, 30)])
 def test_lds_tiles_split_k(M, nleft):
-    """Stage C tiles cut along K, in 64-wide (M = 640) and 128-wide (M = 2047)
-    tiles, against the wave tiles: both sum a few thousand products per element
+    """Stage C tiles cut along K, FP64 in 64-wide tiles and split-BF16 in 128 x 128
+    ones, against the wave tiles: both sum a few thousand products per element
     in FP64, so they agree to 1e-13 of the result's norm.  The split-BF16 tiles
     against that result."""
     from vmps_amd import models
@@ -197,6 +204,7 @@ def test_lds_tiles_split_k(M, nleft):
                           np.random.default_rng(14))
     v = synth.random_vector(pd, 15)
     print("split K", M, "vsize", pd.vsize, flush=True)
+    assert _tiles128(pd) < 256
     H = PivotMatrix2(pd)
     H.set_tiles(big_min64=0, explicit_u=0)
     ref = HxV(H, v)
@@ -211,25 +219,46 @@ def test_lds_tiles_split_k(M, nleft):
     assert np.array_equal(HxV(H, v), out)
 
 
-def test_bf16x3_wide_tiles_at_block_edges():
-    """Stage C's 128 x 256 split-BF16 tiles (pivots of 256 and more 128 x 128
-    tiles), the last of each block 1 to 4 strips of 32 rows and 64 columns wide,
-    against the FP64 wave tiles."""
+@pytest.fixture(scope="module")
+def wide_case():
+    """A pivot of over 256 128 x 128 tiles, the last of each block 1 to 4 strips of 32
+    rows and 32 or 64 columns wide, and its HxV on the FP64 wave tiles."""
     from vmps_amd import models
     W = models.heisenberg_u1_mpo()
     left = [((-1,), 641), ((1,), 700), ((3,), 736), ((5,), 765)]
     right = [((-1,), 769), ((1,), 595), ((3,), 935), ((5,), 1020)]
     pd = synth.make_pivot(W, W, left, right, np.random.default_rng(21))
     v = synth.random_vector(pd, 22)
-    print("wide split-BF16 tiles, vsize", pd.vsize, flush=True)
-    assert pd.vsize >= 256 * 128 * 128
+    assert _tiles128(pd) >= 256
     H = PivotMatrix2(pd)
-    H.set_tiles(big_min64=0, explicit_u=0)
-    ref = HxV(H, v)
-    H.set_precision("bf16x3")
-    H.set_tiles(big_min=1, explicit_u=1)
+    H.set_tiles(wave_edge=32, big_min64=0, explicit_u=0)
+    return pd, v, HxV(H, v)
+
+
+@pytest.mark.parametrize("xu", [1, 0])
+def test_bf16x3_wide_tiles_at_block_edges(wide_case, xu):
+    """Stage C's split-BF16 tiles of such a pivot: 128 x 256 with the explicit stage B,
+    128 x 128 with the fused one, against the FP64 wave tiles."""
+    pd, v, ref = wide_case
+    print("wide split-BF16 tiles, vsize", pd.vsize, xu, flush=True)
+    H = PivotMatrix2(pd, precision="bf16x3")
+    H.set_tiles(big_min=1, explicit_u=xu)
     out = HxV(H, v)
     assert _rel(out, ref) <= BF16X3_RTOL
+    assert np.array_equal(HxV(H, v), out)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 1e-5)])
+@pytest.mark.parametrize("xu", [1, 0])
+def test_128_wide_tiles_at_block_edges(wide_case, precision, tol, xu):
+    """The 128-wide FP64 and FP32 tiles, stage B explicit and fused, against the FP64
+    wave tiles (a few thousand products per element on both sides)."""
+    pd, v, ref = wide_case
+    print("128-wide tiles, vsize", pd.vsize, precision, xu, flush=True)
+    H = PivotMatrix2(pd, precision=precision)
+    H.set_tiles(big_min64=1, explicit_u=xu)
+    out = HxV(H, v)
+    assert _rel(out, ref) <= tol
     assert np.array_equal(HxV(H, v), out)
 
 
