@@ -443,6 +443,11 @@ std::vector<LanczosResult> lanczos_solve_batch(DevPlan& D, BatchKrylov& K, doubl
     // read left some pivot's residual estimate or eigenvalue change at least
     // 100x above its tolerance, the next batch is queued before the host turns
     // to the current one (8 pivots of M <= 256, 120 iterations: 17.5 -> 11.6 ms).
+    // Unlike the single solve's, the look-ahead has no limit on the HxV's work: the
+    // host's part grows with the pivots, and with a limit of 1 GFLOP 16 pivots of
+    // M <= 1024 (2.7 GFLOP) took 234 instead of 205 ms and 8 of M <= 2048 (14.5
+    // GFLOP) 658 instead of 640 ms, with as many HxV: convergence within a batch from
+    // 100x above the tolerance is the exception (a Krylov space that ends).
     // Two instances of the graph and two readback slots alternate.
     constexpr int B = BatchKrylov::kIterBatch;
     const size_t slot_elems = 4 * (size_t)B * P;
