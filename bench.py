@@ -296,6 +296,21 @@ def c2_sweeps(args, sweeps=3):
             "max_truncation_last_sweep": max(r["truncation"][-47:]), "hxv_calls": be.hxv_calls}
 
 
+def split_details(res, path=""):
+    """Takes the lists of records (one per step or sweep) out of `res` and returns
+    them by their path: the result line stays a few thousand characters long, as
+    what keeps only the end of a program's output needs it; the records go to
+    stderr."""
+    details = {}
+    for k in list(res):
+        v = res[k]
+        if isinstance(v, dict):
+            details.update(split_details(v, path + k + "."))
+        elif isinstance(v, list) and (len(v) > 4 or any(isinstance(x, dict) for x in v)):
+            details[path + k] = res.pop(k)
+    return details
+
+
 def dmrg_c60_bench(args):
     import torch
     from vmps_amd import dmrg, lattice, models, synth
@@ -762,6 +777,9 @@ def main():
         res = hxv_bench(args)
         if args.sweeps > 0:
             res["sweeps"] = sweep_bench(args, sweeps=args.sweeps)
+    details = split_details(res)
+    if details:
+        print(json.dumps({"details": details}), file=sys.stderr, flush=True)
     print(json.dumps(res))
 
 
