@@ -254,9 +254,9 @@ vmps_status vmps_plan_get_tiles(const vmps_plan* plan, vmps_tile_config* cfg);
 vmps_status vmps_plan_set_tiles(vmps_plan* plan, const vmps_tile_config* cfg);  /* ms .. n_tried ignored */
 /* Autotuner: times the candidate configurations of the plan's precision
  * (`iters` HxV each on the plan's resident vectors) and keeps the fastest.
- * The candidates follow a rule on the block sizes: on pivots dominated by blocks
- * of 256 and more they are those the plan may start from, whatever was set by
- * hand; on others the current configuration is one of them.
+ * On pivots dominated by blocks of 256 and more there is one candidate, given by
+ * a rule on the block sizes whatever was set by hand; on others the current
+ * configuration is among them.
  * The choice is cached per block-size histogram (the share of the work in
  * classes of block rows x columns) and per precision, so later plans of the
  * same shape take it without timing.  Thread-safe. */

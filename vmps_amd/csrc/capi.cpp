@@ -722,7 +722,7 @@ vmps_status vmps_plan_autotune(vmps_plan* plan, int iters, vmps_tile_config* out
   }
   // Search from the plan's current configuration over the parameters its
   // precision uses (the others stay as they are), keeping the best so far: at
-  // most six candidates; one warm-up call per candidate absorbs its first-call
+  // most five candidates; one warm-up call per candidate absorbs its first-call
   // set-up.
   auto measure = [&](const TileChoice& c) {
     D.retile(c.wave_edge, c.big_min, c.big_min64, c.explicit_u);
